@@ -439,10 +439,10 @@ class Context:
         _check(lib.ck_context_set_option(self._h, CK_OPT_PLAN_AUTOTUNE, int(bool(on))))
 
     def set_bconv_mfma(self, on=True):
-        """BaseConv on the FP64 matrix cores (True), on the int8 matrix cores
-        ("int8"), fused into the forward NTT column pass (False), or None for
-        the default (int8 matrix cores in batched plans, fused in single
-        operations); outputs are identical."""
+        """BaseConv as its own step on the FP64 matrix cores (True) or on the
+        int8 matrix cores ("int8"), or fused with the forward NTT column pass
+        on the int8 matrix cores (False, and the default None); outputs are
+        identical."""
         v = -1 if on is None else 2 if on == "int8" else int(bool(on))
         _check(lib.ck_context_set_option(self._h, CK_OPT_BCONV_MFMA, v))
 

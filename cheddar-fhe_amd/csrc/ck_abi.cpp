@@ -751,7 +751,7 @@ extern "C++" template <typename Build>
 static int build_tuned(const Context &c, Build &build, bool key_dim, int chunk_items,
                        Plan **out) {
   *out = nullptr;
-  if (!c.plan_autotune) return build(c.bconv_mfma < 0 ? 2 : c.bconv_mfma, -1, 0, out);
+  if (!c.plan_autotune) return build(c.bconv_mfma < 0 ? 0 : c.bconv_mfma, -1, 0, out);
   Plan *best = nullptr;
   double best_us = -1.0;
   double us[3] = {-1.0, -1.0, -1.0};

@@ -17,6 +17,7 @@
 #include <mutex>
 
 #include "ck_internal.h"
+#include "ck_i8_arith.h"
 #include "ck_ops.h"
 
 namespace ck {
@@ -128,8 +129,8 @@ int upload(Context &c, T **dptr, const std::vector<T> &h) {
 // plain form (times R^-1 because the reference applies it with a Montgomery
 // product); table[m][i] = centred((prod_{j!=i} s_j) * R^2 mod t_m).
 //
-// ftab holds the same products for the exact FP64 BaseConv fused into the
-// forward NTT: T'[m][i] = (prod_{j!=i} s_j) * R mod t_m (one Montgomery
+// ftab holds the same products for the exact FP64 and int8 BaseConvs:
+// T'[m][i] = (prod_{j!=i} s_j) * R mod t_m (one Montgomery
 // factor: the fused form adds no R^-1) split as hi * 2^16 + lo.
 void bconv_constants(const Context &c, const std::vector<int> &src,
                      const std::vector<int> &dst,
@@ -165,6 +166,17 @@ void bconv_constants(const Context &c, const std::vector<int> &src,
 }
 
 namespace {
+
+// The int8 operand planes (i8::bconv_quad_planes) of a BaseConv table in
+// ftab form.
+int upload_quads(Context &c, int32_t **dptr, const std::vector<double> &ftab, size_t s,
+                 const std::vector<int> &dst) {
+  std::vector<uint32_t> tab(s * dst.size()), dq;
+  for (size_t i = 0; i < tab.size(); i++)
+    tab[i] = (uint32_t)ftab[2 * i] * 65536u + (uint32_t)ftab[2 * i + 1];
+  for (int p : dst) dq.push_back(c.primes[p]);
+  return upload(c, dptr, i8::bconv_quad_planes(tab, (int)s, (int)dst.size(), dq));
+}
 
 // One ModDown flavour from (nm, nt) q primes with naux auxiliary primes to
 // (dm, dt) (ModSwitch.cu:233-303 for the prime ranges, :566-684 for which
@@ -234,6 +246,7 @@ int build_moddown(Context &c, int nm, int nt, int dm, int dt, int naux, int kind
   }
   mp.use_pad = !restore.empty();
   int rc = upload(c, &mp.d_ftab, ftab);
+  if (!rc) rc = upload_quads(c, &mp.d_quads, ftab, src_prime.size(), dst_prime);
   if (rc) return rc;
   mp.valid = true;
   return kOk;
@@ -282,6 +295,7 @@ int build_modup(Context &c, LevelPlan &lp, int nm, int nt, int naux, int pad) {
     bconv_constants(c, src, dst, {}, c1, table, ftab);
     for (int t = s0; t < s1; t++) lp.modup_c1[t] = c1[t - s0];
     int rc = upload(c, &gr.d_ftab, ftab);
+    if (!rc) rc = upload_quads(c, &gr.d_quads, ftab, src.size(), dst);
     if (rc) return rc;
   }
   return kOk;

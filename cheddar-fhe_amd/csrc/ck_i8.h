@@ -76,6 +76,39 @@ void launch_bconv_i8_table(const Context &c, const BconvI8Inst *insts, int n, in
 // kernel-argument form (single operations: no device table)
 void launch_bconv_i8(const Context &c, const BconvI8Launch &L, hipStream_t st);
 
+// ---- BaseConv fused with the forward column stages -------------------------
+
+// Four destination limbs of one BaseConv: S centred int32 source limbs, the
+// quad's operand planes, and for each destination its limb (nullptr past the
+// last one) and prime.
+struct BcolsQuad {
+  const int32_t *src;
+  const int32_t *planes;
+  uint32_t *dst[4];
+  int32_t S;
+  uint8_t prime[4];
+  int64_t pad_;
+};
+static_assert(sizeof(BcolsQuad) == 64, "BcolsQuad is one 64-byte record");
+
+constexpr int kMaxBcolsQuads = 48;  // quads of a kernel-argument launch
+struct BcolsLaunch {
+  BcolsQuad quad[kMaxBcolsQuads];
+};
+
+// The quads of one BaseConv, in destination order; quads = the table's
+// operand planes (bconv_quad_planes).
+void add_bcols_quads(std::vector<BcolsQuad> &out, const int32_t *src, int S,
+                     const int32_t *quads, const std::vector<uint32_t *> &dst,
+                     const std::vector<int> &prime);
+// dst = the column stages of the forward transform of the BaseConv (lazy
+// int32, as the column pass leaves it); limbs / max_s = destinations in all
+// quads / the largest S among them
+void launch_bconv_cols(const Context &c, const BcolsLaunch &L, int n, int limbs, int max_s,
+                       hipStream_t st);
+void launch_bconv_cols_table(const Context &c, const BcolsQuad *quads, int n, int limbs,
+                             int max_s, hipStream_t st);
+
 // The int8 operand planes of a context BaseConv table (a ModUp group's or a
 // ModDown plan's FP64 {hi, lo} table on the device, S sources x D
 // destinations), built on first use from the table's words and kept in the

@@ -46,6 +46,7 @@
 // 16 x 16 tiles (tile_word).
 #include "ck_i8.h"
 #include "ck_i8_arith.h"
+#include "ck_radix16.h"
 
 #include <algorithm>
 #include <cstring>
@@ -461,6 +462,174 @@ __global__ __launch_bounds__(256) void bconv_valu_kernel(const BconvI8Inst *__re
   }
 }
 
+// ---- BaseConv fused with the forward column stages -------------------------
+
+struct BcolsByValue {
+  BcolsLaunch L;
+  __device__ __forceinline__ BcolsQuad quad(int y) const { return L.quad[y]; }
+};
+struct BcolsTable {
+  const BcolsQuad *__restrict__ quads;
+  __device__ __forceinline__ BcolsQuad quad(int y) const {
+    typedef const __attribute__((address_space(4))) BcolsQuad CQuad;
+    CQuad *p = (CQuad *)quads + y;
+    BcolsQuad q;
+    q.src = p->src;
+    q.planes = p->planes;
+    for (int i = 0; i < 4; i++) {
+      q.dst[i] = p->dst[i];
+      q.prime[i] = p->prime[i];
+    }
+    q.S = p->S;
+    return q;
+  }
+};
+
+// BaseConv of 16 rows (16 k apart) at one column for the lane's destination:
+// STEPS products of PER sources a lane (bconv_quad_planes), 16x16x32 for one
+// step of up to 2, else 16x16x64. Sources past S re-read source 0 (their
+// plane bytes are 0), so every load is unconditional and a batch of them is
+// in flight before its first product.
+template <int STEPS, int PER>
+__device__ __forceinline__ void bconv_rows16(const int32_t *src, uint32_t off, int S,
+                                             const int32_t *planes, int lane, double x[16]) {
+  const int g = lane >> 4;
+  const v4i zero = {0, 0, 0, 0};
+  typedef const __attribute__((address_space(1))) char gchar;
+  typedef const __attribute__((address_space(1))) int gint;
+  gchar *base = (gchar *)src;
+  uint32_t o[STEPS][PER];
+#pragma unroll
+  for (int ks = 0; ks < STEPS; ks++)
+#pragma unroll
+    for (int t = 0; t < PER; t++) {
+      const int s = 4 * PER * ks + PER * g + t;
+      o[ks][t] = off + (uint32_t)(s < S ? s : 0) * (4 * kN);
+    }
+  constexpr bool kNarrow = STEPS == 1 && PER <= 2;
+  int64_t a32 = 0;
+  v4i a64[STEPS];
+#pragma unroll
+  for (int ks = 0; ks < STEPS; ks++)
+    if (kNarrow)
+      a32 = ((const int64_t *)planes)[lane];
+    else
+      a64[ks] = ((const v4i *)planes)[64 * ks + lane];
+  constexpr int kB = STEPS * PER <= 2 ? 16 : STEPS * PER <= 4 ? 8 : 4;  // rows of a load batch
+#pragma unroll
+  for (int k0 = 0; k0 < 16; k0 += kB) {
+    int raw[kB][STEPS][PER];
+#pragma unroll
+    for (int k = 0; k < kB; k++)
+#pragma unroll
+      for (int ks = 0; ks < STEPS; ks++)
+#pragma unroll
+        for (int t = 0; t < PER; t++)
+          raw[k][ks][t] = *(gint *)(base + 16384 * (k0 + k) + o[ks][t]);
+#pragma unroll
+    for (int k = 0; k < kB; k++) {
+      v4i d = zero;
+#pragma unroll
+      for (int ks = 0; ks < STEPS; ks++) {
+        int b[4] = {0, 0, 0, 0};
+#pragma unroll
+        for (int t = 0; t < PER; t++) b[t] = pack_c(raw[k][ks][t]);
+        if (kNarrow) {
+          const int64_t b32 = (int64_t)(uint32_t)b[0] | ((int64_t)(uint32_t)b[1] << 32);
+          d = __builtin_amdgcn_mfma_i32_16x16x32_i8(a32, b32, d, 0, 0, 0);
+        } else {
+          d = mfma64(a64[ks], v4i{b[0], b[1], b[2], b[3]}, d);
+        }
+      }
+      x[k0 + k] = combine(d[0], d[1], d[2], d[3]);
+    }
+  }
+}
+
+// ModSwitchMatrixMult (src/core/ModSwitch.cu:23-171) and the column stages of
+// NTTPhase1 (src/core/NTT.cu:231-330) for four destination limbs at once.
+//
+// A workgroup of NC waves owns NC columns of a quad. One matrix product
+// gives a wave the BaseConv of 16 positions for the quad's four
+// destinations, lane group g holding destination g (bconv_quad_planes), so
+// the sources are read once per four destinations and the lanes keep their
+// values in registers for the column stages: lane (g, n) transforms column
+// n % NC, first phase rows rb + 16 k with rb = (16 / NC) wave + n / NC,
+// second phase rows 16 rb + j. The BaseConv sums enter the butterflies
+// unreduced: below 2^46 in magnitude, they stay below 2^47 on the path that
+// is only added to (eight sums of products below 2^31), inside the 2^50 of
+// mulmod_fq and reduce_f.
+//
+// Bound by vector issue: about 850 instructions a wave (512 of them the
+// butterflies) at the 1.9 GHz that FP64 runs at, 83 % of the time of a full
+// chip. The form before it, one limb per workgroup with the BaseConv in FP64
+// on the vector unit, took 1260 and read the sources for every destination:
+// 72 limbs of 8 sources 19.9 -> 16.3 us, 42 of 15 sources 20.8 -> 14.5 us;
+// against BaseConv as its own int8 step and a plain column pass, 4128 limbs
+// of 8 sources 970 -> 739 us. Handing the phases over as int32 (half the
+// LDS, three workgroups per CU) cost 10 % more instructions and 13 % time.
+template <class D, int NC, int WIDTH>
+__global__ __launch_bounds__(64 * NC, 4) void bconv_i8_cols(const D desc, const PrimeTab P,
+                                                           const uint32_t *__restrict__ tw) {
+  constexpr int kRows = 16 / NC;           // row groups rb of one wave
+  constexpr int kShare = 32 / NC;          // column tiles in a 128-byte line
+  constexpr int kTiles = 256 / NC;
+  __shared__ double ldsd[4 * 256 * NC];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int g = lane >> 4, n = lane & 15;
+  // workgroup i runs on XCD i mod 8: the tiles of one line share an XCD
+  const int b = blockIdx.x;
+  const int c0 = (((b & 7) * kShare) | ((b >> 3) & (kShare - 1))) * NC;
+  const BcolsQuad Q = desc.quad(b / kTiles);
+  const int cc = n % NC, rl = n / NC;
+  const int rb = wave * kRows + rl;
+  // the lane's destination
+  uint32_t *dst = g == 0 ? Q.dst[0] : g == 1 ? Q.dst[1] : g == 2 ? Q.dst[2] : Q.dst[3];
+  const int prime = g == 0 ? Q.prime[0] : g == 1 ? Q.prime[1] : g == 2 ? Q.prime[2] : Q.prime[3];
+  const double q = P.qd[prime], qr = P.qr[prime];
+  const ModF m{q, qr};
+  const uint32_t *__restrict__ w = tw + (size_t)prime * kN;
+  uint32_t t1[15], t2[15];
+#pragma unroll
+  for (int s = 0; s < 4; s++)
+#pragma unroll
+    for (int blk = 0; blk < (1 << s); blk++) {
+      t1[(1 << s) - 1 + blk] = w[(1 << s) + blk];
+      t2[(1 << s) - 1 + blk] = w[(16 << s) + (rb << s) + blk];
+    }
+  double x[16];
+  const uint32_t off = 4u * (uint32_t)(rb * 256 + c0 + cc);
+  const int S = Q.S;
+  if (S <= 4)
+    bconv_rows16<1, 1>(Q.src, off, S, Q.planes, lane, x);
+  else if (WIDTH == 0 || S <= 8)
+    bconv_rows16<1, 2>(Q.src, off, S, Q.planes, lane, x);
+  else if (S <= 12)
+    bconv_rows16<1, 3>(Q.src, off, S, Q.planes, lane, x);
+  else if (WIDTH == 1 || S <= 16)
+    bconv_rows16<1, 4>(Q.src, off, S, Q.planes, lane, x);
+  else if constexpr (WIDTH == 2)
+    bconv_rows16<2, 3>(Q.src, off, S, Q.planes, lane, x);
+  ct16(x, t1, q, qr);
+  // hand-off in LDS, rows of NC doubles; within 16 lanes (one LDS cycle of
+  // 128 bytes) the writes cover kRows adjacent rows and the reads kRows rows
+  // 16 apart: rows are swapped by their block number so that both cover all
+  // banks
+  double *tile = ldsd + g * 256 * NC + cc;
+#pragma unroll
+  for (int k = 0; k < 16; k++) tile[(16 * k + (rb ^ (k & (kRows - 1)))) * NC] = x[k];
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 16; j++) x[j] = tile[(16 * rb + (j ^ rl)) * NC];
+  ct16(x, t2, q, qr);
+  if (dst) {
+    typedef __attribute__((address_space(1))) uint32_t guint;
+    guint *o = (guint *)dst + (size_t)(16 * rb) * 256 + c0 + cc;
+#pragma unroll
+    for (int j = 0; j < 16; j++) o[j * 256] = (uint32_t)(int32_t)reduce_f(x[j], m);
+  }
+}
+
 // ---- host tables ------------------------------------------------------------
 
 uint32_t brv_n(uint32_t x, int bits) {
@@ -643,6 +812,67 @@ bool to_i8_inst(const Context &c, const BconvInst &in, BconvI8Inst *out) {
     out->dst_prime[m] = in.dst_prime[m];
   }
   return true;
+}
+
+void add_bcols_quads(std::vector<BcolsQuad> &out, const int32_t *src, int S,
+                     const int32_t *quads, const std::vector<uint32_t *> &dst,
+                     const std::vector<int> &prime) {
+  const size_t D = dst.size();
+  for (size_t d0 = 0; d0 < D; d0 += 4) {
+    BcolsQuad Q;
+    std::memset(&Q, 0, sizeof(Q));
+    Q.src = src;
+    Q.planes = quads + d0 / 4 * i8::bconv_quad_words(S);
+    Q.S = S;
+    for (size_t i = 0; i < 4; i++) {
+      Q.dst[i] = d0 + i < D ? dst[d0 + i] : nullptr;
+      Q.prime[i] = (uint8_t)prime[d0 + i < D ? d0 + i : d0];
+    }
+    out.push_back(Q);
+  }
+}
+
+namespace {
+
+template <class D, int NC>
+void bconv_cols_nc(const Context &c, const D &d, int n, int limbs, int max_s, hipStream_t st) {
+  const dim3 grid(256 / NC * n), block(64 * NC);
+  const uint32_t *tw = c.d_tw_fwd;
+  const char *name = "ntt_fwd_cols+bconv";
+  if (max_s <= 8)
+    launch(c, name, limbs, bconv_i8_cols<D, NC, 0>, grid, block, st, d, c.ptab, tw);
+  else if (max_s <= 16)
+    launch(c, name, limbs, bconv_i8_cols<D, NC, 1>, grid, block, st, d, c.ptab, tw);
+  else
+    launch(c, name, limbs, bconv_i8_cols<D, NC, 2>, grid, block, st, d, c.ptab, tw);
+}
+
+// Columns per workgroup. 8 (two workgroups of 8 waves on a CU) measured
+// faster with up to 8 sources: 72 limbs 16.3 us against 18.3 us with 16
+// columns (one workgroup of 16 waves), 4128 limbs 739 against 815 us; 4
+// columns lose to their 16-byte row segments (72 limbs 20.7 us). With more
+// sources the loads weigh more and whole 64-byte segments win once ten quads
+// fill the chip: 42 limbs of 15 sources 14.5 against 16.9 us, 114 of 12
+// sources 23.5 against 24.5 us; 4 limbs of 9 sources 10.2 against 7.5 us.
+template <class D>
+void bconv_cols(const Context &c, const D &d, int n, int limbs, int max_s, hipStream_t st) {
+  if (n <= 0) return;
+  if (max_s > 8 && n >= 10)
+    bconv_cols_nc<D, 16>(c, d, n, limbs, max_s, st);
+  else
+    bconv_cols_nc<D, 8>(c, d, n, limbs, max_s, st);
+}
+
+}  // namespace
+
+void launch_bconv_cols(const Context &c, const BcolsLaunch &L, int n, int limbs, int max_s,
+                       hipStream_t st) {
+  bconv_cols(c, BcolsByValue{L}, n, limbs, max_s, st);
+}
+
+void launch_bconv_cols_table(const Context &c, const BcolsQuad *quads, int n, int limbs,
+                             int max_s, hipStream_t st) {
+  bconv_cols(c, BcolsTable{quads}, n, limbs, max_s, st);
 }
 
 void launch_bconv_valu_table(const Context &c, const BconvI8Inst *insts, int n, int dsts,

@@ -137,6 +137,47 @@ inline std::vector<int64_t> bconv_i8_planes(const std::vector<uint32_t> &tab, in
   return out;
 }
 
+// Sources that one lane supplies to a k-step of a destination quad's product
+// (S sources over four lane groups; more than 16 take two k-steps).
+inline int bconv_quad_per(int S) { return S <= 16 ? (S + 3) / 4 : (S + 7) / 8; }
+// 32-bit words of the quad's operand planes (bconv_quad_planes).
+inline int bconv_quad_words(int S) { return S <= 8 ? 128 : S <= 16 ? 256 : 512; }
+
+// Operand registers of a BaseConv table in quads of four destinations: row
+// m of an operand is byte plane m & 3 of destination 4 quad + (m >> 2), so
+// that lane group g of the product D[4 g + v][n] receives the four planes of
+// destination 4 quad + g. With per = bconv_quad_per(S), lane l = 16 g + m
+// holds, quad after quad,
+//   S <= 8 (v_mfma_i32_16x16x32_i8): two words, else
+//   (v_mfma_i32_16x16x64_i8): four words for each k-step ks;
+// word t < per is for source 4 per ks + per g + t, byte i of it being digit
+// m & 3 of tab[d][s] 2^(8 i) mod t_d (centred), 0 past D or S; the other
+// words are 0.
+inline std::vector<int32_t> bconv_quad_planes(const std::vector<uint32_t> &tab, int S, int D,
+                                              const std::vector<uint32_t> &dst_q) {
+  const int words = bconv_quad_words(S), quads = (D + 3) / 4;
+  const int per = bconv_quad_per(S), lane_words = S <= 8 ? 2 : 4;
+  std::vector<int32_t> out((size_t)quads * words, 0);
+  for (int d = 0; d < D; d++) {
+    const uint32_t q = dst_q[d];
+    uint32_t p8[4];
+    for (int i = 0; i < 4; i++) p8[i] = powmod_h(2, 8 * i, q);
+    for (int s = 0; s < S; s++) {
+      const int ks = s / (4 * per), g = s / per % 4, t = s % per;
+      uint32_t w[4] = {0, 0, 0, 0};
+      for (int i = 0; i < 4; i++) {
+        const int32_t x = centre_h((uint64_t)tab[(size_t)d * S + s] * p8[i], q);
+        for (int j = 0; j < 4; j++) w[j] |= digit_byte(x, j) << (8 * i);
+      }
+      for (int j = 0; j < 4; j++) {
+        const int lane = 16 * g + 4 * (d & 3) + j;
+        out[(size_t)(d >> 2) * words + ((size_t)ks * 64 + lane) * lane_words + t] = (int32_t)w[j];
+      }
+    }
+  }
+  return out;
+}
+
 }  // namespace i8
 }  // namespace ck
 

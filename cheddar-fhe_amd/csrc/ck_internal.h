@@ -43,12 +43,12 @@ enum NttFlags : int {
   kNttEpiloguePad = 4,      // forward: apply c2 in the epilogue
   kInttCentred = 8,         // inverse: centred int32 output
   kInttLoadProduct = 16,    // inverse: input = src (*) src2 (Montgomery)
-  kNttBconvInput = 32,      // forward: input = BaseConv of bsrc (see below)
   kNttColsOnly = 64,        // forward: column stages only (rows fused later)
+  kNttRowsOnly = 128,       // forward: row stages only (columns done in dst)
 };
 
 // Per-limb fields of a kernel-argument plan, kept together in one record
-// (24 bytes, dword aligned): hipcc for gfx950 has folded a byte-indexed base
+// (20 bytes, dword aligned): hipcc for gfx950 has folded a byte-indexed base
 // into the scalar load of a separate dword array (s_load with a base that
 // is not dword aligned, whose low bits the hardware drops), reading the
 // constant of the neighbouring limb.
@@ -56,47 +56,35 @@ struct NttLimb {
   uint32_t c1, c2, c3;  // plain-form constants (already carry R^-1)
   uint16_t src_limb, dst_limb;
   int16_t src2_limb;
-  uint16_t btab_off;
   uint8_t prime, sel;
-  uint16_t pad_;
 };
-static_assert(sizeof(NttLimb) == 24, "NttLimb is one 24-byte record");
+static_assert(sizeof(NttLimb) == 20, "NttLimb is one 20-byte record");
 
 struct NttLaunch {
   // up to four base pointers per role; limb i uses src[sel & 3],
-  // dst[(sel >> 2) & 3], src2[(sel >> 4) & 3], bsrc[(sel >> 6) & 3]
+  // dst[(sel >> 2) & 3], src2[(sel >> 4) & 3]
   const uint32_t *src[4];
   uint32_t *dst[4];
   const uint32_t *src2[4];
-  // kNttBconvInput: the transform input of limb i is
-  //   sum_j bsrc[j] * T_j  mod q, T_j = B[btab_off + 2j] * 2^16 +
-  //   B[btab_off + 2j + 1], B = btab[(sel >> 6) & 3]
-  // over bs[(sel >> 6) & 3] contiguous centred int32 source limbs
-  // (BaseConv, exact)
-  const int32_t *bsrc[4];
-  const double *btab[4];
-  int bs[4];
   int n;
   int flags;
   NttLimb limb[kMaxLaunchLimbs];
 };
 
 // One limb of a transform pass with every pointer resolved; the form a
-// batched plan keeps in device memory (one table per pass, 64 bytes a limb).
-// src2 == nullptr: no product operand / no kept limb; bsrc == nullptr: no
-// BaseConv input. flags as NttLaunch::flags.
+// batched plan keeps in device memory (one table per pass, 48 bytes a limb).
+// src2 == nullptr: no product operand / no kept limb. flags as
+// NttLaunch::flags.
 struct LimbJob {
   const uint32_t *src;
   uint32_t *dst;
   const uint32_t *src2;
-  const int32_t *bsrc;
-  const double *btab;  // this output limb's row: bs x {hi, lo}
   uint32_t c1, c2, c3;
-  uint16_t prime, bs;
+  uint16_t prime, pad0_;
   int32_t flags;
-  int32_t pad_;
+  int32_t pad1_;
 };
-static_assert(sizeof(LimbJob) == 64, "LimbJob is one 64-byte record");
+static_assert(sizeof(LimbJob) == 48, "LimbJob is one 48-byte record");
 
 // source limbs of one BaseConv: up to 5 terminal + 12 auxiliary primes in
 // the reference's parameter files (bootparam_35.json); 24 keeps every exact
@@ -117,7 +105,8 @@ struct ModDownPlan {
   std::vector<uint32_t> pad;   // epilogue padding (plain)
   std::vector<uint32_t> inv_prod;  // epilogue (prod src)^-1 (plain)
   bool use_pad = false;
-  double *d_ftab = nullptr;    // dst_len x src_len x {hi, lo}, see NttLaunch
+  double *d_ftab = nullptr;    // dst_len x src_len x {hi, lo} 16-bit halves
+  int32_t *d_quads = nullptr;  // int8 operand planes by destination quad
 };
 
 struct ModUpGroup {
@@ -125,6 +114,7 @@ struct ModUpGroup {
   std::vector<int> dst_limb;    // limb index in the (num_q + alpha) output
   std::vector<int> dst_prime;   // global prime
   double *d_ftab = nullptr;     // dst x src x {hi, lo}
+  int32_t *d_quads = nullptr;   // int8 operand planes by destination quad
 };
 
 struct LevelPlan {
@@ -169,10 +159,9 @@ struct Context {
   int short_naux = 0;
   uint32_t *d_p_prod_short = nullptr;
 
-  // BaseConv as its own step on the matrix cores instead of fused into the
-  // forward column pass: 1 FP64 matrix cores everywhere, 2 int8 matrix
-  // cores everywhere, 0 fused everywhere, -1 (default) int8 matrix cores in
-  // batched plans and fused in single operations (measured fastest)
+  // BaseConv as its own step on the matrix cores instead of fused with the
+  // forward column pass: 1 FP64 matrix cores, 2 int8 matrix cores, 0 or -1
+  // (default) fused (measured fastest for single operations and batches)
   int bconv_mfma = -1;
   // int8 operand planes of the BaseConv tables, by FP64 table (built on
   // first use, freed with the context)
@@ -274,10 +263,9 @@ void bconv_constants(const Context &c, const std::vector<int> &src,
 void launch_ntt_fwd(const Context &ctx, const NttLaunch &L, hipStream_t st);
 void launch_intt(const Context &ctx, const NttLaunch &L, hipStream_t st);
 // table form: n jobs in device memory; flags_any = OR of the jobs' flags
-// (names the launch for profiling); max_bs = the largest BaseConv source
-// count among the jobs (selects the column kernel's instantiation)
+// (selects the passes and names the launch for profiling)
 void launch_ntt_fwd_table(const Context &ctx, const LimbJob *jobs, int n,
-                          int flags_any, int max_bs, hipStream_t st);
+                          int flags_any, hipStream_t st);
 void launch_intt_table(const Context &ctx, const LimbJob *jobs, int n,
                        int flags_any, hipStream_t st);
 

@@ -21,19 +21,17 @@
 //     registers (32 KiB of LDS: four workgroups and more fit a CU).
 // Each thread runs two radix-16 register phases on 16 values; the hand-off
 // between the two phases keeps the lazy doubles in an LDS tile (row tiles
-// use an XOR swizzle so both phase layouts are free of bank conflicts; the
-// column pass's BaseConv stages its int32 output in the same LDS words
-// first). Twiddles are read once per workgroup phase as u32
+// use an XOR swizzle so both phase layouts are free of bank conflicts).
+// Twiddles are read once per workgroup phase as u32
 // and issued before the data loads. Butterflies use the exact FP64 modular
 // product of ck_arith.h with lazy ranges (integer doubles below 2^40); the
 // intermediate between the two passes of a transform is stored as a lazy
 // int32 in (-0.75 q, 0.75 q) and only final outputs are made canonical.
 // Each thread writes a phase's results back to exactly the LDS words it read
 // for that phase, so only the hand-offs between threads need a barrier.
-#include <algorithm>
-
 #include "ck_elem.h"
 #include "ck_internal.h"
+#include "ck_radix16.h"
 
 namespace ck {
 namespace {
@@ -45,28 +43,6 @@ constexpr int kRowTiles = 256 / kRowTile;     // per limb
 constexpr int kColThreads = 256;
 constexpr int kColTile = 16;                  // columns per column workgroup
 constexpr int kColTiles = 256 / kColTile;     // per limb
-
-// forward radix-16 (4 CT stages), element index bits high to low; twiddle
-// slot (1 << s) - 1 + blk for sub-stage s
-__device__ __forceinline__ void ct16(double x[16], const uint32_t tw[15],
-                                     double q, double qr) {
-#pragma unroll
-  for (int s = 0; s < 4; s++) {
-    const int half = 8 >> s;
-#pragma unroll
-    for (int blk = 0; blk < (1 << s); blk++) {
-      const double w = (double)tw[(1 << s) - 1 + blk];
-#pragma unroll
-      for (int j = 0; j < half; j++) {
-        double &a = x[blk * 2 * half + j];
-        double &b = x[blk * 2 * half + j + half];
-        const double r = mulmod_fq(b, w, q, qr);
-        b = a - r;
-        a = a + r;
-      }
-    }
-  }
-}
 
 // ct16 with the twiddles kept in LDS, slot i of this thread at
 // tws[i * kRowThreads + threadIdx.x] (conflict-free): for a loop that runs
@@ -92,28 +68,6 @@ __device__ __forceinline__ void ct16_lds(double x[16], const uint32_t *tws,
   }
 }
 
-// inverse radix-16 (4 GS stages), element index bits low to high; twiddle
-// slot 16 - (16 >> u) + blk for sub-stage u
-__device__ __forceinline__ void gs16(double x[16], const uint32_t tw[15],
-                                     double q, double qr) {
-#pragma unroll
-  for (int u = 0; u < 4; u++) {
-    const int half = 1 << u;
-#pragma unroll
-    for (int blk = 0; blk < (8 >> u); blk++) {
-      const double w = (double)tw[16 - (16 >> u) + blk];
-#pragma unroll
-      for (int j = 0; j < half; j++) {
-        double &a = x[blk * 2 * half + j];
-        double &b = x[blk * 2 * half + j + half];
-        const double d = a - b;
-        a = a + b;
-        b = mulmod_fq(d, w, q, qr);
-      }
-    }
-  }
-}
-
 // Row-tile LDS index: row rl, in-row offset b, XOR swizzle of the low nibble
 // by the high nibble (both b = t + 16k and b = 16t + j patterns hit 16
 // distinct banks).
@@ -129,15 +83,11 @@ struct JobByValue {
   __device__ __forceinline__ LimbJob job(int y) const {
     const NttLimb &R = L.limb[y];
     const int sel = R.sel;
-    const int b = (sel >> 6) & 3;
     LimbJob J;
     J.src = L.src[sel & 3] + (size_t)R.src_limb * kN;
     J.dst = L.dst[(sel >> 2) & 3] + (size_t)R.dst_limb * kN;
     const uint32_t *s2 = L.src2[(sel >> 4) & 3];
     J.src2 = (s2 && R.src2_limb >= 0) ? s2 + (size_t)R.src2_limb * kN : nullptr;
-    J.bsrc = L.bsrc[b];
-    J.btab = L.btab[b] ? L.btab[b] + R.btab_off : nullptr;
-    J.bs = (uint16_t)L.bs[b];
     J.c1 = R.c1;
     J.c2 = R.c2;
     J.c3 = R.c3;
@@ -158,13 +108,10 @@ struct JobTable {
     J.src = p->src;
     J.dst = p->dst;
     J.src2 = p->src2;
-    J.bsrc = p->bsrc;
-    J.btab = p->btab;
     J.c1 = p->c1;
     J.c2 = p->c2;
     J.c3 = p->c3;
     J.prime = p->prime;
-    J.bs = p->bs;
     J.flags = p->flags;
     return J;
   }
@@ -199,119 +146,6 @@ __device__ __forceinline__ ColTile col_tile() {
   return ColTile{(int)(blockIdx.x >> 4), t * kColTile};
 }
 
-// BaseConv computed straight into the column tile (ModSwitchMatrixMult,
-// src/core/ModSwitch.cu:23-171, in exact FP64): for each coefficient,
-// y = sum_j v_j * T_j mod t over bs centred int32 source limbs, with
-// T_j = hi_j * 2^16 + lo_j so every partial sum stays an exact double
-// (|v| < 2^30, hi < 2^15, lo < 2^16: |sum v hi| < 2^50 and
-// |sum v lo| < 2^51 for bs <= 24).
-// Output: int32 tile [256][16] in LDS, 16-byte source loads.
-//
-// MS (>= bs) bounds the unrolled source loop. All loads
-// of a batch of up to KB sources are issued unconditionally before the first
-// product (sources past bs re-read source 0 and get zero table entries): a
-// load inside a branch that also consumes it would be waited for at once,
-// one memory latency per source. VEC coefficients per load: 4 (16 bytes),
-// or 2 for MS >= 12, whose 24 or 32 table doubles leave fewer registers.
-template <int MS, int VEC, int KB = 8>
-__device__ __forceinline__ void bconv_cols_ms(const int32_t *bsrc, int bs,
-                                              const double *tab, int c0,
-                                              const ModF &m, int32_t *lds) {
-  typedef int32_t ivec __attribute__((ext_vector_type(VEC)));
-  constexpr int kRowLanes = kColTile / VEC;                 // lanes per row
-  constexpr int kIters = 256 * kColTile / (kColThreads * VEC);
-  // the table row is read-only and uniform: scalar loads (constant space)
-  typedef const __attribute__((address_space(4))) double cdouble;
-  cdouble *ctab = (cdouble *)tab;
-  double th[MS], tl[MS];
-#pragma unroll
-  for (int j = 0; j < MS; j++) {
-    const int jj = j < bs ? j : 0;
-    const double h = ctab[2 * jj], l = ctab[2 * jj + 1];
-    th[j] = j < bs ? h : 0.0;
-    tl[j] = j < bs ? l : 0.0;
-  }
-#pragma unroll
-  for (int i = 0; i < kIters; i++) {
-    const int idx = kColThreads * i + threadIdx.x;  // VEC-word chunk index
-    const int r = idx / kRowLanes, cv = (idx % kRowLanes) * VEC;
-    const int32_t *p = bsrc + r * 256 + c0 + cv;
-    double sh[VEC], sl[VEC];
-#pragma unroll
-    for (int e = 0; e < VEC; e++) sh[e] = sl[e] = 0.0;
-#pragma unroll
-    for (int j0 = 0; j0 < MS; j0 += KB) {
-      constexpr int kB = MS < KB ? MS : KB;
-      ivec v[kB];
-#pragma unroll
-      for (int j = 0; j < kB; j++) {
-        if (j0 + j >= MS) break;  // static after unrolling
-        const int jj = j0 + j < bs ? j0 + j : 0;
-        v[j] = *reinterpret_cast<const ivec *>(p + (size_t)jj * kN);
-      }
-#pragma unroll
-      for (int j = 0; j < kB; j++) {
-        if (j0 + j >= MS) break;
-#pragma unroll
-        for (int e = 0; e < VEC; e++) {
-          const double vv = (double)v[j][e];
-          sh[e] = __builtin_fma(vv, th[j0 + j], sh[e]);
-          sl[e] = __builtin_fma(vv, tl[j0 + j], sl[e]);
-        }
-      }
-    }
-    ivec o;
-#pragma unroll
-    for (int e = 0; e < VEC; e++) {
-      const double big = sh[e] * 65536.0;  // exact (power-of-two scale)
-      const double k = __builtin_rint(big * m.qinv);
-      o[e] = (int32_t)reduce_f(__builtin_fma(-k, m.q, big) + sl[e], m);
-    }
-    *reinterpret_cast<ivec *>(lds + r * kColTile + cv) = o;
-  }
-}
-
-// bs is uniform per workgroup: one branch-free body per source bound.
-// WIDTH 1: the instantiation for launches with 10..16 sources, whose
-// 12- and 13-source bodies keep 16-byte loads at four waves per SIMD (at
-// five they only fit with 8-byte loads); WIDTH 2: 17..24 sources (terminal
-// plus auxiliary primes of a rescale), at three waves per SIMD
-template <int WIDTH>
-__device__ __forceinline__ void bconv_cols_to_lds(const int32_t *bsrc, int bs,
-                                                  const double *tab, int c0,
-                                                  const ModF &m,
-                                                  int32_t *lds) {
-  // exact bodies for the common counts (alpha and 1 + alpha of the shipped
-  // parameter sets: 8, 9, 12, 13), bounded bodies otherwise
-  switch (bs) {
-    case 8: bconv_cols_ms<8, 4>(bsrc, bs, tab, c0, m, lds); return;
-    case 9: bconv_cols_ms<9, 4, 5>(bsrc, bs, tab, c0, m, lds); return;
-    case 12:
-      if (WIDTH >= 1)
-        bconv_cols_ms<12, 4, 6>(bsrc, bs, tab, c0, m, lds);
-      else
-        bconv_cols_ms<12, 2>(bsrc, bs, tab, c0, m, lds);
-      return;
-    case 13:
-      if (WIDTH >= 1)
-        bconv_cols_ms<13, 4, 5>(bsrc, bs, tab, c0, m, lds);
-      else
-        bconv_cols_ms<13, 2>(bsrc, bs, tab, c0, m, lds);
-      return;
-    default: break;
-  }
-  if (bs <= 4)
-    bconv_cols_ms<4, 4>(bsrc, bs, tab, c0, m, lds);
-  else if (bs <= 8)
-    bconv_cols_ms<8, 4>(bsrc, bs, tab, c0, m, lds);
-  else if (bs <= 12)
-    bconv_cols_ms<12, 2>(bsrc, bs, tab, c0, m, lds);
-  else if (WIDTH < 2 || bs <= 16)
-    bconv_cols_ms<16, 2>(bsrc, bs, tab, c0, m, lds);
-  else if constexpr (WIDTH == 2)
-    bconv_cols_ms<kMaxBconvSrc, 2, 6>(bsrc, bs, tab, c0, m, lds);
-}
-
 // Final value of an element: canonical u32, or lazy int32 in
 // (-0.75 q, 0.75 q) for a pass-1 intermediate that pass 2 reads back.
 __device__ __forceinline__ int32_t lazy_i32(double x, const ModF &m) {
@@ -321,12 +155,10 @@ __device__ __forceinline__ int32_t lazy_i32(double x, const ModF &m) {
 // ---------------------------------------------------------------------------
 // Forward, column stages s = 0..7 -> lazy int32 intermediate
 // ---------------------------------------------------------------------------
-template <class D, int WIDTH>
-__global__ __launch_bounds__(kColThreads, 5 - WIDTH) void ntt_fwd_cols(
+template <class D>
+__global__ __launch_bounds__(kColThreads, 5) void ntt_fwd_cols(
     const D desc, const PrimeTab P, const uint32_t *__restrict__ tw) {
-  // int32 BaseConv tile [256][16] aliased with the double exchange tile
   __shared__ double ldsd[256 * kColTile];
-  int32_t *lds = reinterpret_cast<int32_t *>(ldsd);
   const ColTile ct = col_tile();
   const int c0 = ct.c0;
   const LimbJob J = desc.job(ct.y);
@@ -339,28 +171,17 @@ __global__ __launch_bounds__(kColThreads, 5 - WIDTH) void ntt_fwd_cols(
   // phase 1 twiddles psi_rev[2^s + blk] (uniform), phase 2 psi_rev[2^(4+s)
   // + rb 2^s + blk]
   uint32_t t1[15], t2[15];
-  auto load_twiddles = [&]() {
 #pragma unroll
-    for (int s = 0; s < 4; s++)
+  for (int s = 0; s < 4; s++)
 #pragma unroll
-      for (int blk = 0; blk < (1 << s); blk++) {
-        t1[(1 << s) - 1 + blk] = w[(1 << s) + blk];
-        t2[(1 << s) - 1 + blk] = w[(16 << s) + (rb << s) + blk];
-      }
-  };
-  // phase 1 holds rows rb + 16 k of column c0 + cc
+    for (int blk = 0; blk < (1 << s); blk++) {
+      t1[(1 << s) - 1 + blk] = w[(1 << s) + blk];
+      t2[(1 << s) - 1 + blk] = w[(16 << s) + (rb << s) + blk];
+    }
+  // phase 1 holds rows rb + 16 k of column c0 + cc: canonical residues
+  // (< 2^31) or a lazy signed BaseConv output, as int32
   double x[16];
-  if (J.flags & kNttBconvInput) {
-    // twiddles after the BaseConv, whose loads need the registers
-    bconv_cols_to_lds<WIDTH>(J.bsrc, J.bs, J.btab, c0, m, lds);
-    load_twiddles();
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < 16; k++) x[k] = (double)lds[(rb + 16 * k) * kColTile + cc];
-    __syncthreads();  // the staging words are reused by the double tile
-  } else {
-    load_twiddles();
-    // canonical residues (< 2^31) or a lazy signed BaseConv output: int32
+  {
     const int32_t *__restrict__ g =
         reinterpret_cast<const int32_t *>(J.src) + c0 + cc;
 #pragma unroll
@@ -826,9 +647,6 @@ __global__ __launch_bounds__(kRowThreads, 2) void key_rows_table_kernel(
   key_rows_body(np, P, it.A, tw, y, ldsd, tws);
 }
 
-const char *fwd_cols_name(int flags) {
-  return (flags & kNttBconvInput) ? "ntt_fwd_cols+bconv" : "ntt_fwd_cols";
-}
 const char *fwd_rows_name(int flags) {
   return (flags & kNttModDownEpilogue) ? "ntt_fwd_rows+epilogue" : "ntt_fwd_rows";
 }
@@ -837,17 +655,10 @@ const char *inv_rows_name(int flags) {
 }
 
 template <class D>
-void fwd_passes(const Context &ctx, const D &d, int n, int flags, int max_bs,
-                hipStream_t st) {
-  if ((flags & kNttBconvInput) && max_bs > 16)
-    launch(ctx, fwd_cols_name(flags), n, ntt_fwd_cols<D, 2>, dim3(kColTiles * n),
-           dim3(kColThreads), st, d, ctx.ptab, (const uint32_t *)ctx.d_tw_fwd);
-  else if ((flags & kNttBconvInput) && max_bs > 9)
-    launch(ctx, fwd_cols_name(flags), n, ntt_fwd_cols<D, 1>, dim3(kColTiles * n),
-           dim3(kColThreads), st, d, ctx.ptab, (const uint32_t *)ctx.d_tw_fwd);
-  else
-    launch(ctx, fwd_cols_name(flags), n, ntt_fwd_cols<D, 0>, dim3(kColTiles * n),
-           dim3(kColThreads), st, d, ctx.ptab, (const uint32_t *)ctx.d_tw_fwd);
+void fwd_passes(const Context &ctx, const D &d, int n, int flags, hipStream_t st) {
+  if (!(flags & kNttRowsOnly))
+    launch(ctx, "ntt_fwd_cols", n, ntt_fwd_cols<D>, dim3(kColTiles * n), dim3(kColThreads),
+           st, d, ctx.ptab, (const uint32_t *)ctx.d_tw_fwd);
   if (!(flags & kNttColsOnly))
     launch(ctx, fwd_rows_name(flags), n, ntt_fwd_rows<D>, dim3(kRowTiles, n),
            dim3(kRowThreads), st, d, ctx.ptab, (const uint32_t *)ctx.d_tw_fwd);
@@ -868,9 +679,7 @@ void inv_passes(const Context &ctx, const D &d, int n, int flags,
 // on dst (with the optional ModDown epilogue).
 void launch_ntt_fwd(const Context &ctx, const NttLaunch &L, hipStream_t st) {
   if (L.n <= 0) return;
-  int max_bs = 0;
-  for (int i = 0; i < 4; i++) max_bs = std::max(max_bs, L.bs[i]);
-  fwd_passes(ctx, JobByValue{L}, L.n, L.flags, max_bs, st);
+  fwd_passes(ctx, JobByValue{L}, L.n, L.flags, st);
 }
 
 // Inverse NTT of L.n limbs: row stages into dst, then column stages in
@@ -881,9 +690,9 @@ void launch_intt(const Context &ctx, const NttLaunch &L, hipStream_t st) {
 }
 
 void launch_ntt_fwd_table(const Context &ctx, const LimbJob *jobs, int n,
-                          int flags_any, int max_bs, hipStream_t st) {
+                          int flags_any, hipStream_t st) {
   if (n <= 0) return;
-  fwd_passes(ctx, JobTable{jobs}, n, flags_any, max_bs, st);
+  fwd_passes(ctx, JobTable{jobs}, n, flags_any, st);
 }
 
 void launch_key_rows(const Context &ctx, const EwNp &np, const KeyAccumArgs &A,

@@ -9,7 +9,8 @@
 // copy and no synchronisation.
 //
 // Fusions relative to the reference's kernel sequence (results identical):
-//   * BaseConv runs inside the forward NTT's column pass (ModUp and ModDown),
+//   * BaseConv and the forward NTT's column stages are one pass (ModUp and
+//     ModDown),
 //   * HMult's Tensor product a1 (*) a2 is formed while the ModUp INTT loads,
 //     and d0 = b1 (*) b2, d1 = b1 (*) a2 + a1 (*) b2 inside the key inner
 //     product's P * (d0, d1) fold,
@@ -54,11 +55,11 @@ int slot_of(T *arr, int &n, T ptr) {
 int ImmediateSink::pass(bool forward, int flags,
                         const std::vector<PassJob> &jobs) {
   NttLaunch L;
-  int ns = 0, nd = 0, n2 = 0, nb = 0;
+  int ns = 0, nd = 0, n2 = 0;
   auto reset = [&]() {
     std::memset(&L, 0, sizeof(L));
     L.flags = flags;
-    ns = nd = n2 = nb = 0;
+    ns = nd = n2 = 0;
   };
   auto flush = [&]() {
     if (L.n == 0) return;
@@ -74,25 +75,13 @@ int ImmediateSink::pass(bool forward, int flags,
       int a = slot_of(L.src, ns, j.src);
       int b = slot_of(L.dst, nd, j.dst);
       int s2 = slot_of(L.src2, n2, j.src2);
-      // BaseConv sources and table go together
-      int bc = -1;
-      for (int i = 0; i < nb; i++)
-        if (L.bsrc[i] == j.bsrc && L.btab[i] == j.btab && L.bs[i] == j.bs)
-          bc = i;
-      if (bc < 0 && nb < 4) {
-        L.bsrc[nb] = j.bsrc;
-        L.btab[nb] = j.btab;
-        L.bs[nb] = j.bs;
-        bc = nb++;
-      }
-      if (a >= 0 && b >= 0 && s2 >= 0 && bc >= 0 && L.n < kMaxLaunchLimbs) {
+      if (a >= 0 && b >= 0 && s2 >= 0 && L.n < kMaxLaunchLimbs) {
         NttLimb &R = L.limb[L.n++];
         R.prime = (uint8_t)j.prime;
-        R.sel = (uint8_t)(a | (b << 2) | (s2 << 4) | (bc << 6));
+        R.sel = (uint8_t)(a | (b << 2) | (s2 << 4));
         R.src_limb = (uint16_t)j.src_limb;
         R.dst_limb = (uint16_t)j.dst_limb;
         R.src2_limb = (int16_t)(j.src2 ? j.src2_limb : -1);
-        R.btab_off = (uint16_t)j.btab_off;
         R.c1 = j.c1;
         R.c2 = j.c2;
         R.c3 = j.c3;
@@ -131,6 +120,21 @@ int ImmediateSink::bconv(const std::vector<BconvInst> &insts) {
     L.n = (int)std::min<size_t>(kMaxBconvInst, insts.size() - i);
     for (int k = 0; k < L.n; k++) L.inst[k] = insts[i + k];
     launch_bconv_mfma(c_, L, st_);
+  }
+  return launch_status("bconv");
+}
+
+int ImmediateSink::bconv_cols(const std::vector<BcolsQuad> &quads) {
+  for (size_t i = 0; i < quads.size(); i += kMaxBcolsQuads) {
+    BcolsLaunch L;
+    const int n = (int)std::min<size_t>(kMaxBcolsQuads, quads.size() - i);
+    int limbs = 0, max_s = 0;
+    for (int k = 0; k < n; k++) {
+      L.quad[k] = quads[i + k];
+      max_s = std::max(max_s, quads[i + k].S);
+      for (uint32_t *d : quads[i + k].dst) limbs += d != nullptr;
+    }
+    launch_bconv_cols(c_, L, n, limbs, max_s, st_);
   }
   return launch_status("bconv");
 }
@@ -244,11 +248,12 @@ int op_modup(const Context &c, int level, uint32_t *dst, const uint32_t *src,
     int rc = s.pass(false, kInttCentred | (prod2 ? kInttLoadProduct : 0), jobs);
     if (rc) return rc;
   }
-  // 2. BaseConv of each group, on the matrix cores or fused into the
-  // forward NTT of its outputs
+  // 2. BaseConv of each group, as its own step or fused with the column
+  // stages of the forward NTT of its outputs
   const bool mfma = s.mfma_bconv();
   std::vector<PassJob> jobs;
   std::vector<BconvInst> insts;
+  std::vector<BcolsQuad> quads;
   for (int g = 0; g < lp.beta; g++) {
     const ModUpGroup &gr = lp.groups[g];
     if (gr.s1 <= gr.s0) continue;
@@ -267,26 +272,25 @@ int op_modup(const Context &c, int level, uint32_t *dst, const uint32_t *src,
         I.dst_prime[m] = (uint8_t)gr.dst_prime[m];
       }
       insts.push_back(I);
+    } else {
+      std::vector<uint32_t *> out;
+      for (int t : gr.dst_limb) out.push_back(dst + ((size_t)g * tot + t) * kLimb);
+      add_bcols_quads(quads, bsrc, sl, gr.d_quads, out, gr.dst_prime);
     }
+    if (!mfma && cols_only) continue;
     for (size_t m = 0; m < gr.dst_limb.size(); m++) {
       PassJob j;
       j.src = dst;
       j.dst = dst;
       j.src_limb = j.dst_limb = g * tot + gr.dst_limb[m];
-      if (!mfma) {
-        j.bsrc = bsrc;
-        j.btab = gr.d_ftab;
-        j.bs = sl;
-        j.btab_off = 2 * (int)m * sl;
-      }
       j.prime = gr.dst_prime[m];
       j.c1 = 1;
       jobs.push_back(j);
     }
   }
-  int rc = mfma ? s.bconv(insts) : kOk;
-  if (!rc)
-    rc = s.pass(true, (mfma ? 0 : kNttBconvInput) | (cols_only ? kNttColsOnly : 0), jobs);
+  int rc = mfma ? s.bconv(insts) : s.bconv_cols(quads);
+  if (!rc && (mfma || !cols_only))
+    rc = s.pass(true, mfma ? (cols_only ? kNttColsOnly : 0) : kNttRowsOnly, jobs);
   if (rc) return rc;
   if (copy_own) {
     for (int g = 0; g < lp.beta; g++) {
@@ -336,11 +340,12 @@ int op_moddown(const Context &c, int level, int kind, int npoly,
     int rc = s.pass(false, kInttCentred, jobs);
     if (rc) return rc;
   }
-  // 2. BaseConv (matrix cores, or fused into the forward NTT), 3. epilogue
-  // in the row pass
+  // 2. BaseConv (its own step, or fused with the forward column stages), 3.
+  // epilogue in the row pass
   const bool mfma = s.mfma_bconv();
   std::vector<PassJob> jobs;
   std::vector<BconvInst> insts;
+  std::vector<BcolsQuad> quads;
   for (int k = 0; k < npoly; k++) {
     const int32_t *bsrc =
         reinterpret_cast<const int32_t *>(v + (size_t)k * mp->src_len * kLimb);
@@ -357,6 +362,10 @@ int op_moddown(const Context &c, int level, int kind, int npoly,
         I.dst_prime[y] = (uint8_t)mp->dst_prime[y];
       }
       insts.push_back(I);
+    } else {
+      std::vector<uint32_t *> out;
+      for (int y = 0; y < mp->dst_len; y++) out.push_back(dst[k] + (size_t)y * kLimb);
+      add_bcols_quads(quads, bsrc, mp->src_len, mp->d_quads, out, mp->dst_prime);
     }
     for (int y = 0; y < mp->dst_len; y++) {
       PassJob j;
@@ -365,12 +374,6 @@ int op_moddown(const Context &c, int level, int kind, int npoly,
       j.src_limb = j.dst_limb = y;
       j.src2 = src[k];
       j.src2_limb = mp->src2_limb[y];
-      if (!mfma) {
-        j.bsrc = bsrc;
-        j.btab = mp->d_ftab;
-        j.bs = mp->src_len;
-        j.btab_off = 2 * y * mp->src_len;
-      }
       j.prime = mp->dst_prime[y];
       j.c1 = 1;
       j.c2 = mp->pad[y];
@@ -378,12 +381,10 @@ int op_moddown(const Context &c, int level, int kind, int npoly,
       jobs.push_back(j);
     }
   }
-  if (mfma) {
-    int rc = s.bconv(insts);
-    if (rc) return rc;
-  }
+  int rc = mfma ? s.bconv(insts) : s.bconv_cols(quads);
+  if (rc) return rc;
   return s.pass(true,
-                (mfma ? 0 : kNttBconvInput) | kNttModDownEpilogue |
+                (mfma ? 0 : kNttRowsOnly) | kNttModDownEpilogue |
                     (mp->use_pad ? kNttEpiloguePad : 0),
                 jobs);
 }

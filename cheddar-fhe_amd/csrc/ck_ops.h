@@ -9,6 +9,7 @@
 
 #include "ck_bconv.h"
 #include "ck_elem.h"
+#include "ck_i8.h"
 
 namespace ck {
 
@@ -21,10 +22,6 @@ struct PassJob {
   int dst_limb = 0;
   const uint32_t *src2 = nullptr;  // product operand / kept limb
   int src2_limb = -1;              // -1: none
-  const int32_t *bsrc = nullptr;   // BaseConv sources (bs contiguous limbs)
-  const double *btab = nullptr;    // BaseConv table of the destination set
-  int bs = 0;
-  int btab_off = 0;                // row of this limb in btab (doubles)
   int prime = 0;
   uint32_t c1 = 0, c2 = 0, c3 = 0;
 };
@@ -37,7 +34,9 @@ class Sink {
   virtual int copy(uint32_t *dst, const uint32_t *src, size_t words) = 0;
   // BaseConv instances on the matrix cores (outputs: lazy int32 limbs)
   virtual int bconv(const std::vector<BconvInst> &insts) = 0;
-  // whether ops should emit bconv() steps rather than fused BaseConv passes
+  // BaseConv and the forward column stages of its outputs as one pass
+  virtual int bconv_cols(const std::vector<BcolsQuad> &quads) = 0;
+  // whether ops should emit bconv() steps rather than bconv_cols() ones
   virtual bool mfma_bconv() const = 0;
   // key switches: the ModUp's forward row stages fused with the key inner
   // product (key_rows) or a row pass plus key_accum
@@ -58,6 +57,7 @@ class ImmediateSink : public Sink {
   int pass(bool forward, int flags, const std::vector<PassJob> &jobs) override;
   int copy(uint32_t *dst, const uint32_t *src, size_t words) override;
   int bconv(const std::vector<BconvInst> &insts) override;
+  int bconv_cols(const std::vector<BcolsQuad> &quads) override;
   bool mfma_bconv() const override { return c_.bconv_mfma == 1 || c_.bconv_mfma == 2; }
   int key_accum(const EwNp &np, const KeyAccumArgs &A) override;
   int key_rows(const EwNp &np, const KeyAccumArgs &A) override;

@@ -55,15 +55,11 @@ int PlanSink::pass(bool forward, int flags, const std::vector<PassJob> &jobs) {
     J.dst = j.dst + (size_t)j.dst_limb * kLimb;
     J.src2 = (j.src2 && j.src2_limb >= 0) ? j.src2 + (size_t)j.src2_limb * kLimb
                                           : nullptr;
-    J.bsrc = j.bsrc;
-    J.btab = j.btab ? j.btab + j.btab_off : nullptr;
-    J.bs = (uint16_t)j.bs;
     J.c1 = j.c1;
     J.c2 = j.c2;
     J.c3 = j.c3;
     J.prime = (uint16_t)j.prime;
     J.flags = flags;
-    s.max_bs = std::max(s.max_bs, j.bs);
     s.jobs.push_back(J);
   }
   return kOk;
@@ -86,6 +82,12 @@ int PlanSink::bconv(const std::vector<BconvInst> &insts) {
   }
   PlanStage &s = stage(PlanStage::kBconv);
   s.bc.insert(s.bc.end(), insts.begin(), insts.end());
+  return kOk;
+}
+
+int PlanSink::bconv_cols(const std::vector<BcolsQuad> &quads) {
+  PlanStage &s = stage(PlanStage::kBconvCols);
+  s.bq.insert(s.bq.end(), quads.begin(), quads.end());
   return kOk;
 }
 
@@ -128,13 +130,11 @@ int ew_prime(const EwNp &np, int y) {
 // Jobs of one step are independent, so their order is free: grouping them by
 // prime lets consecutive workgroups share the twiddle table (transforms) or
 // the key limb (key products, whose keys every item shares) in cache instead
-// of each item fetching it from HBM.
-// A BaseConv-input pass is the exception: its output limbs of one
-// polynomial re-read the same source tiles, so they stay together.
+// of each item fetching it from HBM. The quads of a fused BaseConv are not
+// reordered: those of one polynomial re-read the same source tiles.
 void order_by_prime(PlanStage &s) {
-  if (!(s.flags_any & kNttBconvInput))
-    std::stable_sort(s.jobs.begin(), s.jobs.end(),
-                     [](const LimbJob &a, const LimbJob &b) { return a.prime < b.prime; });
+  std::stable_sort(s.jobs.begin(), s.jobs.end(),
+                   [](const LimbJob &a, const LimbJob &b) { return a.prime < b.prime; });
   const bool ka = s.kind == PlanStage::kKeyAccum || s.kind == PlanStage::kKeyRows;
   auto prime_of = [&](const EwJob &j) {
     return ka ? ew_prime(s.ka[j.item].np, j.y) : ew_prime(s.bs[j.item].np, j.y);
@@ -166,6 +166,7 @@ int plan_finish(Plan &p, bool mismatch) {
     if (!rc) rc = upload_vec(p, &s.d_bc, s.bc);
     if (!rc) rc = upload_vec(p, &s.d_n8, s.n8);
     if (!rc) rc = upload_vec(p, &s.d_bi, s.bi);
+    if (!rc) rc = upload_vec(p, &s.d_bq, s.bq);
     if (rc) return rc;
   }
   return kOk;
@@ -212,7 +213,7 @@ int plan_run(const Plan &p, hipStream_t st) {
   for (const PlanStage &s : p.stages) {
     switch (s.kind) {
       case PlanStage::kFwd:
-        launch_ntt_fwd_table(c, s.d_jobs, (int)s.jobs.size(), s.flags_any, s.max_bs, st);
+        launch_ntt_fwd_table(c, s.d_jobs, (int)s.jobs.size(), s.flags_any, st);
         break;
       case PlanStage::kInv:
         launch_intt_table(c, s.d_jobs, (int)s.jobs.size(), s.flags_any, st);
@@ -244,6 +245,15 @@ int plan_run(const Plan &p, hipStream_t st) {
           launch_bconv_i8_table(c, s.d_bi, (int)s.bi.size(), dsts, max_s, max_d, st);
         else
           launch_bconv_valu_table(c, s.d_bi, (int)s.bi.size(), dsts, max_s, st);
+        break;
+      }
+      case PlanStage::kBconvCols: {
+        int limbs = 0, max_s = 1;
+        for (const BcolsQuad &Q : s.bq) {
+          for (uint32_t *d : Q.dst) limbs += d != nullptr;
+          max_s = std::max(max_s, Q.S);
+        }
+        launch_bconv_cols_table(c, s.d_bq, (int)s.bq.size(), limbs, max_s, st);
         break;
       }
       case PlanStage::kBconv: {
@@ -295,7 +305,7 @@ double plan_time_us(const Plan &p, int reps) {
 int plan_launches(const Plan &p) {
   int n = 0;
   for (const PlanStage &s : p.stages)
-    n += ((s.kind == PlanStage::kFwd && !(s.flags_any & kNttColsOnly)) ||
+    n += ((s.kind == PlanStage::kFwd && !(s.flags_any & (kNttColsOnly | kNttRowsOnly))) ||
           s.kind == PlanStage::kInv)
              ? 2
              : 1;

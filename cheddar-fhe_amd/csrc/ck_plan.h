@@ -12,10 +12,10 @@ struct PlanStage {
   enum Kind {
     kFwd, kInv, kKeyAccum, kKeyRows, kBsFused, kBconv,
     kNtt8Cols, kNtt8Rows,   // int8 matrix-core transform passes
-    kBconvI8, kBconvValu    // BaseConv on the int8 matrix cores / vector unit
+    kBconvI8, kBconvValu,   // BaseConv on the int8 matrix cores / vector unit
+    kBconvCols              // BaseConv fused with the forward column stages
   } kind = kFwd;
   int flags_any = 0;
-  int max_bs = 0;  // largest BaseConv source count among the jobs
   std::vector<LimbJob> jobs;
   std::vector<KeyAccumItem> ka;
   std::vector<BsFusedItem> bs;
@@ -23,11 +23,13 @@ struct PlanStage {
   std::vector<BconvInst> bc;
   std::vector<Ntt8Job> n8;      // kNtt8Cols / kNtt8Rows
   std::vector<BconvI8Inst> bi;  // kBconvI8 / kBconvValu
+  std::vector<BcolsQuad> bq;    // kBconvCols
   int blocks = 16;              // int8 passes: 16-column / 16-row blocks per workgroup
   LimbJob *d_jobs = nullptr;
   BconvInst *d_bc = nullptr;
   Ntt8Job *d_n8 = nullptr;
   BconvI8Inst *d_bi = nullptr;
+  BcolsQuad *d_bq = nullptr;
   KeyAccumItem *d_ka = nullptr;
   BsFusedItem *d_bs = nullptr;
   EwJob *d_ew = nullptr;
@@ -75,6 +77,7 @@ class PlanSink : public Sink {
   int pass(bool forward, int flags, const std::vector<PassJob> &jobs) override;
   int copy(uint32_t *dst, const uint32_t *src, size_t words) override;
   int bconv(const std::vector<BconvInst> &insts) override;
+  int bconv_cols(const std::vector<BcolsQuad> &quads) override;
   int key_accum(const EwNp &np, const KeyAccumArgs &A) override;
   int key_rows(const EwNp &np, const KeyAccumArgs &A) override;
   int bs_fused(const EwNp &np, const BsFusedArgs &A) override;

@@ -390,11 +390,11 @@ int ck_plan_destroy(ck_plan *plan);
 
 /* ---- Options ------------------------------------------------------------------ */
 /* CK_OPT_BCONV_MFMA: 1 runs every BaseConv (ModUp, ModDown, Rescale) on the
- * FP64 matrix cores as its own step, 2 on the int8 matrix cores (residues
- * and table split into bytes), 0 fuses it into the forward NTT's column
- * pass, -1 (default) uses the int8 matrix cores for batched plans and the
- * fused form for single operations; results are identical. No reference counterpart (the
- * reference's kFuseModDownEpilogue-style compile-time switches,
+ * FP64 matrix cores as its own step, 2 on the int8 matrix cores as its own
+ * step (residues and table split into bytes), 0 fuses it, on the int8 matrix
+ * cores, with the forward NTT's column pass; -1 (default) is 0. Results are
+ * identical. No reference counterpart (the reference's
+ * kFuseModDownEpilogue-style compile-time switches,
  * include/core/Parameter.h:13-20, select kernel fusions the same way). */
 #define CK_OPT_BCONV_MFMA 1
 /* CK_OPT_PLAN_AUTOTUNE: 1 makes ck_plan_hmult / ck_plan_hrot_hoisted build
