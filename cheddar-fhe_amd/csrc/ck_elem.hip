@@ -38,6 +38,10 @@ __device__ __forceinline__ uint4 ld4(const uint32_t *p) {
   const v4u32 v = *(const gv4u32 *)p;
   return make_uint4(v.x, v.y, v.z, v.w);
 }
+__device__ __forceinline__ uint4 ld4nt(const uint32_t *p) {
+  const v4u32 v = __builtin_nontemporal_load((const gv4u32 *)p);
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
 __device__ __forceinline__ void st4(uint32_t *p, uint4 v) {
   const v4u32 w = {v.x, v.y, v.z, v.w};
   *(gv4u32 *)p = w;
@@ -419,137 +423,152 @@ __global__ __launch_bounds__(kThreads) void key_accum_table_kernel(
 }
 
 // Hoisted baby step (BSFusedKernel, src/extension/Hoist.cu:21-78): the ModUp
-// values of 4 coefficients are loaded once and reused by every rotation;
-// each rotation's products are accumulated and scattered to the
-// automorphism's positions d = brv17((brv17(x) + 1) g^-1 - 1). The grid is
-// XCD-aware: the 64 workgroups of one limb share an XCD (workgroup i runs on
-// XCD i mod 8), so the partial-line scatter writes of a limb merge in one
-// L2.
+// values of a row (256 coefficients, four per lane of one wave) are loaded
+// once and reused by every rotation; each rotation's products are summed in
+// 64 bits, reduced once and stored at the automorphism's positions
+// d = brv17((brv17(x) + 1) g^-1 - 1).
+//
+// The automorphism maps whole rows: the low nine bits of brv17(x) + 1 hold
+// the row of x alone, and multiplying by g^-1 mod 2^17 keeps them apart from
+// the rest. So a wave permutes its row through LDS and writes it as one
+// contiguous kilobyte. Scattering the words to memory instead left the merging
+// of partial lines to an L2 that the outputs of eight rotations overflow, and
+// one Montgomery product per term cost about ten instructions.
+//
+// Workgroups: 64 chunks of four rows a limb, chunk c on XCD c mod 8; in an
+// XCD windows of eight limbs run chunk by chunk, so that the items of a batch,
+// whose jobs are ordered by prime, read a key's lines from one L2 together.
+//
+// Bound by memory: 8 rotations of 8 ciphertexts at 8..24 limbs (193 limbs)
+// took 502 us with the scatter and take 320 us, 7 rotations of one at 59 limbs
+// (1.1 GB of keys and outputs) 235 -> 210 us.
 constexpr int kBsBlocksPerLimb = 65536 / (kThreads * kVec);
+constexpr int kBsWindow = 8;
 
-__device__ __forceinline__ void bs_fused_body(const EwNp &np, const PrimeTab &P,
-                                              const BsFusedArgs &A, int y,
-                                              int k) {
+struct BsPlace {
+  int job, chunk;
+};
+__device__ __forceinline__ BsPlace bs_place() {
+  const int i = blockIdx.x >> 3, per = kBsBlocksPerLimb / 8 * kBsWindow;
+  const int w = i % per;
+  return BsPlace{(i / per) * kBsWindow + w % kBsWindow,
+                 (w / kBsWindow) * 8 + (int)(blockIdx.x & 7)};
+}
+
+// NG >= ngroups bounds the groups; FULL: equal to it; NT: non-temporal key
+// loads
+template <int NG, bool FULL, bool NT>
+__device__ __forceinline__ void bs_fused_row(const EwNp &np, const PrimeTab &P,
+                                             const BsFusedArgs &A, int y, int k,
+                                             uint32_t *row) {
   const int p = ew_prime(np, y);
   const uint32_t q = P.q[p];
   const int32_t qinv = P.qinv[p];
   const size_t my = (size_t)y * 65536 + k;
   const size_t kp = (size_t)p * 65536 + k;
   const size_t tot_stride = (size_t)np.num_total * 65536;
-  // register arrays: every loop over groups is unrolled to the static bound
-  // loads of all groups issued before any use (a load in a branch that
-  // also uses it is waited for at once): exact bodies per count up to 4
-  uint32_t mu[kMaxBsGroups][4];
-  auto load_mu = [&](auto ng_tag, int g0) {
-    constexpr int NG = decltype(ng_tag)::value;
-    uint4 v[NG];
-#pragma unroll
-    for (int b = 0; b < NG; b++) {
-      const int gi = g0 + b;
-      const bool own = (y >= A.own0[gi] && y < A.own1[gi]);
-      const uint32_t *src = own ? A.x : A.modup + (size_t)A.group[gi] * tot_stride;
-      v[b] = ld4(src + my);
-    }
-#pragma unroll
-    for (int b = 0; b < NG; b++) {
-      mu[g0 + b][0] = v[b].x;
-      mu[g0 + b][1] = v[b].y;
-      mu[g0 + b][2] = v[b].z;
-      mu[g0 + b][3] = v[b].w;
-    }
-  };
   const int ng = A.ngroups;
-  const int nfull = ng >= 4 ? 4 : 0;  // kMaxBsGroups = 8: at most two batches
-  if (nfull) load_mu(IntC<4>{}, 0);
-  switch (ng - nfull) {
-    case 1: load_mu(IntC<1>{}, nfull); break;
-    case 2: load_mu(IntC<2>{}, nfull); break;
-    case 3: load_mu(IntC<3>{}, nfull); break;
-    case 4: load_mu(IntC<4>{}, nfull); break;
-    default: break;
+  // groups past ngroups re-read group 0 and count as zero: all loads are
+  // unconditional and in flight together
+  uint32_t mu[NG][4];
+#pragma unroll
+  for (int b = 0; b < NG; b++) {
+    const int gi = FULL || b < ng ? b : 0;
+    const bool own = (y >= A.own0[gi] && y < A.own1[gi]);
+    const uint32_t *src = own ? A.x : A.modup + (size_t)A.group[gi] * tot_stride;
+    const uint4 v = ld4(src + my);
+    const bool use = FULL || b < ng;
+    mu[b][0] = use ? v.x : 0u;
+    mu[b][1] = use ? v.y : 0u;
+    mu[b][2] = use ? v.z : 0u;
+    mu[b][3] = use ? v.w : 0u;
   }
-  uint32_t pb[4] = {0, 0, 0, 0};
+  uint64_t pb[4] = {0, 0, 0, 0};
   if (y < np.num_q) {
     const uint32_t pp = ld1(A.p_prod + p);
     const uint4 v = ld4(A.b + my);
-    pb[0] = mont_mul(pp, v.x, q, qinv);
-    pb[1] = mont_mul(pp, v.y, q, qinv);
-    pb[2] = mont_mul(pp, v.z, q, qinv);
-    pb[3] = mont_mul(pp, v.w, q, qinv);
+    const uint32_t V[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int i = 0; i < 4; i++) pb[i] = (uint64_t)pp * V[i];
   }
-  uint32_t d[4];
+  uint32_t *rb = row, *ra = row + 256;
+  const int lane4 = (int)(threadIdx.x & 63) * 4;
   for (int r = 0; r < A.nrot; r++) {
-    uint32_t rb[4] = {pb[0], pb[1], pb[2], pb[3]}, ra[4] = {0, 0, 0, 0};
-    auto keys = [&](auto ng_tag, int g0) {
-      constexpr int NG = decltype(ng_tag)::value;
-      uint4 kb[NG], ka[NG];
+    uint4 kb[NG], ka[NG];
 #pragma unroll
-      for (int b = 0; b < NG; b++) {
-        kb[b] = ld4(A.key_b[r][g0 + b] + kp);
-        ka[b] = ld4(A.key_a[r][g0 + b] + kp);
-      }
+    for (int b = 0; b < NG; b++) {
+      const int gi = FULL || b < ng ? b : 0;
+      kb[b] = NT ? ld4nt(A.key_b[r][gi] + kp) : ld4(A.key_b[r][gi] + kp);
+      ka[b] = NT ? ld4nt(A.key_a[r][gi] + kp) : ld4(A.key_a[r][gi] + kp);
+    }
+    uint64_t sb[4] = {pb[0], pb[1], pb[2], pb[3]}, sa[4] = {0, 0, 0, 0};
 #pragma unroll
-      for (int b = 0; b < NG; b++) {
-        const uint32_t KB[4] = {kb[b].x, kb[b].y, kb[b].z, kb[b].w};
-        const uint32_t KA[4] = {ka[b].x, ka[b].y, ka[b].z, ka[b].w};
+    for (int b = 0; b < NG; b++) {
+      const uint32_t KB[4] = {kb[b].x, kb[b].y, kb[b].z, kb[b].w};
+      const uint32_t KA[4] = {ka[b].x, ka[b].y, ka[b].z, ka[b].w};
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-          rb[i] = add_mod(rb[i], mont_mul(mu[g0 + b][i], KB[i], q, qinv), q);
-          ra[i] = add_mod(ra[i], mont_mul(mu[g0 + b][i], KA[i], q, qinv), q);
+      for (int i = 0; i < 4; i++) {
+        sb[i] += (uint64_t)mu[b][i] * KB[i];
+        sa[i] += (uint64_t)mu[b][i] * KA[i];
+        if (b & 1 || b == NG - 1) {
+          sb[i] = sum_fold(sb[i], q);
+          sa[i] = sum_fold(sa[i], q);
         }
       }
-    };
-    if (nfull) keys(IntC<4>{}, 0);
-    switch (ng - nfull) {
-      case 1: keys(IntC<1>{}, nfull); break;
-      case 2: keys(IntC<2>{}, nfull); break;
-      case 3: keys(IntC<3>{}, nfull); break;
-      case 4: keys(IntC<4>{}, nfull); break;
-      default: break;
     }
     const uint32_t g = A.ginv[r];
+    uint32_t d = 0;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       const uint32_t e = (__brev((uint32_t)(k + i)) >> 15) + 1u;
-      d[i] = __brev((e * g - 1u) & 0x1FFFFu) >> 15;
+      d = __brev((e * g - 1u) & 0x1FFFFu) >> 15;
+      rb[d & 255] = sum_reduce(sb[i], q, qinv);
+      ra[d & 255] = sum_reduce(sa[i], q, qinv);
     }
-    uint32_t *ob = A.out_b[r] + (size_t)y * 65536;
-    uint32_t *oa = A.out_a[r] + (size_t)y * 65536;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      st1(ob + d[i], rb[i]);
-      st1(oa + d[i], ra[i]);
-    }
+    __builtin_amdgcn_wave_barrier();  // one wave's LDS accesses run in order
+    const uint4 ob = *reinterpret_cast<const uint4 *>(rb + lane4);
+    const uint4 oa = *reinterpret_cast<const uint4 *>(ra + lane4);
+    __builtin_amdgcn_wave_barrier();
+    const size_t o = (size_t)y * 65536 + (d & 0xFF00u) + lane4;
+    st4(A.out_b[r] + o, ob);
+    st4(A.out_a[r] + o, oa);
   }
 }
 
-// limb slot of workgroup blockIdx.x for `nlimbs` limbs (XCD-aware order);
-// returns -1 for the padding workgroups of the last group of 8 limbs
-__device__ __forceinline__ int bs_limb(int nlimbs, int &chunk) {
-  const int xcd = blockIdx.x & 7;
-  const int j = blockIdx.x >> 3;
-  chunk = j % kBsBlocksPerLimb;
-  const int y = (j / kBsBlocksPerLimb) * 8 + xcd;
-  return y < nlimbs ? y : -1;
+template <bool NT>
+__device__ __forceinline__ void bs_fused_body(const EwNp &np, const PrimeTab &P,
+                                              const BsFusedArgs &A, int y, int chunk,
+                                              uint32_t *lds) {
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int k = chunk * kThreads * kVec + (int)threadIdx.x * kVec;
+  uint32_t *row = lds + 512 * wave;
+  switch (A.ngroups) {
+    case 1: bs_fused_row<1, true, NT>(np, P, A, y, k, row); break;
+    case 2: bs_fused_row<2, true, NT>(np, P, A, y, k, row); break;
+    case 3: bs_fused_row<3, true, NT>(np, P, A, y, k, row); break;
+    case 4: bs_fused_row<4, true, NT>(np, P, A, y, k, row); break;
+    default: bs_fused_row<kMaxBsGroups, false, NT>(np, P, A, y, k, row); break;
+  }
 }
 
+template <bool NT>
 __global__ __launch_bounds__(kThreads) void bs_fused_kernel(
     const EwNp np, const PrimeTab P, const BsFusedArgs A) {
-  int chunk;
-  const int y = bs_limb(np.num_total, chunk);
-  if (y < 0) return;
-  bs_fused_body(np, P, A, y, (chunk * kThreads + threadIdx.x) * kVec);
+  __shared__ __align__(16) uint32_t lds[2 * kThreads * kVec];
+  const BsPlace at = bs_place();
+  if (at.job >= np.num_total) return;
+  bs_fused_body<NT>(np, P, A, at.job, at.chunk, lds);
 }
 
 __global__ __launch_bounds__(kThreads) void bs_fused_table_kernel(
     const BsFusedItem *__restrict__ items, const EwJob *__restrict__ jobs,
     int njobs, const PrimeTab P) {
-  int chunk;
-  const int j = bs_limb(njobs, chunk);
-  if (j < 0) return;
-  const EwJob jb = jobs[j];
+  __shared__ __align__(16) uint32_t lds[2 * kThreads * kVec];
+  const BsPlace at = bs_place();
+  if (at.job >= njobs) return;
+  const EwJob jb = jobs[at.job];
   const BsFusedItem &it = items[jb.item];
-  bs_fused_body(it.np, P, it.A, jb.y, (chunk * kThreads + threadIdx.x) * kVec);
+  bs_fused_body<false>(it.np, P, it.A, jb.y, at.chunk, lds);
 }
 
 // Permute (ElementWise.cu:370-391): dst[i] = src[brv17((brv17(i)+1) g - 1)]
@@ -770,13 +789,19 @@ int launch_copy(const Context &ctx, void *dst, const void *src, size_t bytes,
 }
 
 static int bs_grid(int nlimbs) {
-  return ((nlimbs + 7) / 8) * 8 * kBsBlocksPerLimb;
+  return (nlimbs + kBsWindow - 1) / kBsWindow * kBsWindow * kBsBlocksPerLimb;
 }
 
 void launch_bs_fused(const Context &ctx, const EwNp &np, const BsFusedArgs &A,
                      hipStream_t st) {
   if (np.num_total <= 0 || A.nrot <= 0) return;
-  launch(ctx, "bs_fused", np.num_total, bs_fused_kernel,
+  // keys that pass by once and outgrow half of the 256 MB last-level cache
+  // are read non-temporally (59 limbs, 7 rotations, 826 MB of keys: 229 ->
+  // 210 us); a batch's items share theirs (320 against 481 us with
+  // non-temporal loads)
+  const size_t key_bytes = (size_t)A.nrot * 2 * A.ngroups * np.num_total * 65536 * 4;
+  launch(ctx, "bs_fused", np.num_total,
+         key_bytes > (128u << 20) ? bs_fused_kernel<true> : bs_fused_kernel<false>,
          dim3(bs_grid(np.num_total)), dim3(kThreads), st, np, ctx.ptab, A);
 }
 
