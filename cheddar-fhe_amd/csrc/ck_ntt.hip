@@ -439,19 +439,24 @@ __global__ __launch_bounds__(kColThreads, 5) void intt_cols(
 // the column pass (lazy int32 in `modup`), runs the row stages in registers
 // and multiplies the 16 values each thread holds by the key limbs, so the
 // ModUp output never goes back to memory in NTT form. A group's own limbs
-// are the ModUp source itself (x, or the Tensor product a1 (*) a2). In the
-// Montgomery convention of the stored data the result is
-//   acc_x[y] = R^-1 (sum_g m_g * key_x,g + fold_x)  mod q,
-// fold_b = P * b1 b2 (HMult) or P R * add_b, fold_a likewise, which is
-// exactly the key_accum kernel's sum of Montgomery products; here every
-// product is an exact FP64 modular product of lazy values and one product by
-// R^-1 ends the sum.
+// are the ModUp source itself (x, or the Tensor product a1 (*) a2). The
+// row outputs are made canonical and the products summed in 64 bits
+// (sum_fold, sum_reduce), as Montgomery products of the stored data:
+//   acc_x[y] = R^-1 (sum_g m_g * key_x,g + P R * fold_x)  mod q,
+// fold_b = d0 = b1 (*) b2 (HMult) or add_b, fold_a likewise, which is exactly
+// the key_accum kernel's sum.
+//
+// Bound by memory: the keys, 50 MB for 32 limbs and three groups, pass by
+// once, 111 MB in all at least. With every product reduced by itself in FP64
+// the kernel issued about 2540 vector instructions where it now has 1690:
+// 32 limbs 26.8 -> 23.4 us, 382 limbs of a batch 218 -> 195 us.
 template <class Args>
 __device__ __forceinline__ void key_rows_body(const EwNp &np, const PrimeTab &P,
                                               Args &A, const uint32_t *tw, int y,
                                               double *ldsd, uint32_t *tws) {
   const int p = y < np.num_q ? np.q_prime0 + y : np.aux_prime0 + (y - np.num_q);
   const double q = P.qd[p], qr = P.qr[p];
+  const ModF m{q, qr};
   const uint32_t qu = P.q[p];
   const int32_t qinv = P.qinv[p];
   const uint32_t *__restrict__ w = tw + (size_t)p * kN;
@@ -465,8 +470,6 @@ __device__ __forceinline__ void key_rows_body(const EwNp &np, const PrimeTab &P,
   const int kl = y < np.num_q ? A.key_q0 + y : A.key_aux0 + (y - np.num_q);
   const size_t kp = (size_t)kl * kN + off;
   const bool tens = A.use_tensor && y < np.num_q;
-  // R^-1 and P = (P R) R^-1 as plain residues (Montgomery reductions)
-  const double rinv = (double)mont_reduce(1, qu, qinv), rinvq = rinv * qr;
 
   // row-stage twiddles (as ntt_fwd_rows), parked in LDS for the group loop:
   // slot i of this thread at tws[i * 256 + tid] (phase 1: 0..14, 2: 15..29);
@@ -480,9 +483,9 @@ __device__ __forceinline__ void key_rows_body(const EwNp &np, const PrimeTab &P,
           w[(4096 << s) + (r << (4 + s)) + (t16 << s) + blk];
     }
 
-  double sb[16], sa[16];
+  uint64_t sb[16], sa[16];
 #pragma unroll
-  for (int j = 0; j < 16; j++) sb[j] = sa[j] = 0.0;
+  for (int j = 0; j < 16; j++) sb[j] = sa[j] = 0;
   // the column-pass tile of the next group that needs the row stages is
   // loaded one group ahead (into `pre`), so its latency overlaps the
   // current group's arithmetic
@@ -514,36 +517,34 @@ __device__ __forceinline__ void key_rows_body(const EwNp &np, const PrimeTab &P,
       kb[i] = reinterpret_cast<const uint4 *>(kbp)[i];
       ka[i] = reinterpret_cast<const uint4 *>(kap)[i];
     }
-    double x[16];
+    uint32_t v[16];
     if (own) {
       if (tens) {
-        // d2 = a1 (*) a2 = a1 a2 R^-1
+        // d2 = a1 (*) a2
         const uint4 *a1 = reinterpret_cast<const uint4 *>(A.tensor[1] + my);
         const uint4 *a2 = reinterpret_cast<const uint4 *>(A.tensor[3] + my);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-          const uint4 u = a1[i], v = a2[i];
-          const uint32_t U[4] = {u.x, u.y, u.z, u.w}, V[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-          for (int e = 0; e < 4; e++) {
-            const double vd = (double)V[e];
-            const double t = mulmod_fq((double)U[e], vd, q, qr);
-            x[4 * i + e] = mulmod_f(t, rinv, rinvq, q);
-          }
+          const uint4 u = a1[i], w2 = a2[i];
+          v[4 * i + 0] = sum_reduce((uint64_t)u.x * w2.x, qu, qinv);
+          v[4 * i + 1] = sum_reduce((uint64_t)u.y * w2.y, qu, qinv);
+          v[4 * i + 2] = sum_reduce((uint64_t)u.z * w2.z, qu, qinv);
+          v[4 * i + 3] = sum_reduce((uint64_t)u.w * w2.w, qu, qinv);
         }
       } else {
         const uint4 *xs = reinterpret_cast<const uint4 *>(A.x + my);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
           const uint4 u = xs[i];
-          x[4 * i + 0] = (double)u.x;
-          x[4 * i + 1] = (double)u.y;
-          x[4 * i + 2] = (double)u.z;
-          x[4 * i + 3] = (double)u.w;
+          v[4 * i + 0] = u.x;
+          v[4 * i + 1] = u.y;
+          v[4 * i + 2] = u.z;
+          v[4 * i + 3] = u.w;
         }
       }
     } else {
       // gi == pg: its tile is in `pre`; start the next one
+      double x[16];
 #pragma unroll
       for (int k = 0; k < 16; k++) x[k] = (double)pre[k];
       pg = next_rows_group(gi + 1);
@@ -556,23 +557,32 @@ __device__ __forceinline__ void key_rows_body(const EwNp &np, const PrimeTab &P,
 #pragma unroll
       for (int j = 0; j < 16; j++) x[j] = ldsd[rlds(rl, 16 * t16 + j)];
       ct16_lds(x, tws + 15 * kRowThreads, q, qr);
+#pragma unroll
+      for (int j = 0; j < 16; j++) v[j] = canon_f(x[j], m);
     }
+    const bool fold = gi & 1;  // two products between folds
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       const uint32_t KB[4] = {kb[i].x, kb[i].y, kb[i].z, kb[i].w};
       const uint32_t KA[4] = {ka[i].x, ka[i].y, ka[i].z, ka[i].w};
 #pragma unroll
       for (int e = 0; e < 4; e++) {
-        const double b = (double)KB[e], a = (double)KA[e];
-        sb[4 * i + e] += mulmod_fq(x[4 * i + e], b, q, qr);
-        sa[4 * i + e] += mulmod_fq(x[4 * i + e], a, q, qr);
+        sb[4 * i + e] += (uint64_t)v[4 * i + e] * KB[e];
+        sa[4 * i + e] += (uint64_t)v[4 * i + e] * KA[e];
+      }
+    }
+    if (fold) {
+#pragma unroll
+      for (int j = 0; j < 16; j++) {
+        sb[j] = sum_fold(sb[j], qu);
+        sa[j] = sum_fold(sa[j], qu);
       }
     }
   }
 
-  // the P fold on q limbs
+  // the P fold on q limbs: one more product (at most two since a fold)
+  const uint32_t pp = y < np.num_q ? A.p_prod[p] : 0u;
   if (tens) {
-    const double pq = (double)mont_reduce(A.p_prod[p], qu, qinv), pqq = pq * qr;
     const uint4 *b1 = reinterpret_cast<const uint4 *>(A.tensor[0] + my);
     const uint4 *a1 = reinterpret_cast<const uint4 *>(A.tensor[1] + my);
     const uint4 *b2 = reinterpret_cast<const uint4 *>(A.tensor[2] + my);
@@ -584,29 +594,27 @@ __device__ __forceinline__ void key_rows_body(const EwNp &np, const PrimeTab &P,
       const uint32_t B2[4] = {u2.x, u2.y, u2.z, u2.w}, A2[4] = {v2.x, v2.y, v2.z, v2.w};
 #pragma unroll
       for (int e = 0; e < 4; e++) {
-        const double db1 = (double)B1[e], da1 = (double)A1[e];
-        const double db2 = (double)B2[e], da2 = (double)A2[e];
-        const double d0 = mulmod_fq(db1, db2, q, qr);
-        const double d1 = mulmod_fq(db1, da2, q, qr) + mulmod_fq(da1, db2, q, qr);
-        sb[4 * i + e] += mulmod_f(d0, pq, pqq, q);
-        sa[4 * i + e] += mulmod_f(d1, pq, pqq, q);
+        const uint32_t d0 = sum_reduce((uint64_t)B1[e] * B2[e], qu, qinv);
+        const uint32_t d1 =
+            sum_reduce((uint64_t)B1[e] * A2[e] + (uint64_t)A1[e] * B2[e], qu, qinv);
+        sb[4 * i + e] += (uint64_t)pp * d0;
+        sa[4 * i + e] += (uint64_t)pp * d1;
       }
     }
   } else if (y < np.num_q && (A.add_b || A.add_a)) {
-    const double pp = (double)A.p_prod[p], ppq = pp * qr;
 #pragma unroll
     for (int i = 0; i < 4; i++) {
       if (A.add_b) {
         const uint4 u = reinterpret_cast<const uint4 *>(A.add_b + my)[i];
         const uint32_t U[4] = {u.x, u.y, u.z, u.w};
 #pragma unroll
-        for (int e = 0; e < 4; e++) sb[4 * i + e] += mulmod_f((double)U[e], pp, ppq, q);
+        for (int e = 0; e < 4; e++) sb[4 * i + e] += (uint64_t)pp * U[e];
       }
       if (A.add_a) {
         const uint4 u = reinterpret_cast<const uint4 *>(A.add_a + my)[i];
         const uint32_t U[4] = {u.x, u.y, u.z, u.w};
 #pragma unroll
-        for (int e = 0; e < 4; e++) sa[4 * i + e] += mulmod_f((double)U[e], pp, ppq, q);
+        for (int e = 0; e < 4; e++) sa[4 * i + e] += (uint64_t)pp * U[e];
       }
     }
   }
@@ -618,8 +626,8 @@ __device__ __forceinline__ void key_rows_body(const EwNp &np, const PrimeTab &P,
     uint32_t vb[4], va[4];
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-      vb[e] = canon_small(mulmod_f(sb[4 * i + e], rinv, rinvq, q), q);
-      va[e] = canon_small(mulmod_f(sa[4 * i + e], rinv, rinvq, q), q);
+      vb[e] = sum_reduce(sum_fold(sb[4 * i + e], qu), qu, qinv);
+      va[e] = sum_reduce(sum_fold(sa[4 * i + e], qu), qu, qinv);
     }
     ob[i] = make_uint4(vb[0], vb[1], vb[2], vb[3]);
     oa[i] = make_uint4(va[0], va[1], va[2], va[3]);
