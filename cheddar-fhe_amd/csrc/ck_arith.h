@@ -98,7 +98,8 @@ __device__ __forceinline__ uint64_t sum_fold(uint64_t a, uint32_t q) {
 // a < q 2^32 -> a 2^-32 mod q, canonical
 __device__ __forceinline__ uint32_t sum_reduce(uint64_t a, uint32_t q, int32_t qinv) {
   const uint32_t t = (uint32_t)a * (uint32_t)qinv;
-  const uint32_t r = (uint32_t)(a >> 32) - __umulhi(t, q);  // (-q, q)
+  const uint32_t m = (uint32_t)(((uint64_t)t * q) >> 32);
+  const uint32_t r = (uint32_t)(a >> 32) - m;  // (-q, q)
   const uint32_t u = r + q;
   return r < u ? r : u;
 }
