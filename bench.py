@@ -112,7 +112,8 @@ _KERNELS = ("ntt_fwd_cols", "intt_cols", "ntt_fwd_rows", "intt_rows", "key_accum
             "bconv_mfma_table", "key_rows", "key_rows_table", "gs_accum")
 # int8 matrix-core kernels (batched plans): labelled by workgroup count, since
 # their workgroups per limb depend on the plan's blocks per workgroup
-_I8_KERNELS = ("ntt8_cols", "ntt8_rows", "bconv_i8", "bconv_valu", "bconv_i8_cols")
+_I8_KERNELS = ("ntt8_cols", "ntt8_rows", "ntt1p_fwd", "ntt1p_inv", "bconv_i8", "bconv_valu",
+               "bconv_i8_cols")
 
 
 def _limbs(short, grid_x, grid_y, wg_x):

@@ -28,9 +28,12 @@ COMMON = [
 
 # per-file flags: the int8 matrix-core kernels keep their MFMA results in
 # ordinary VGPRs (the default allocation parks them in accumulation
-# registers and copies every result back with v_accvgpr_read)
+# registers and copies every result back with v_accvgpr_read); the one-pass
+# transforms index register arrays in loops that must unroll whole, past the
+# compiler's default size limit
 EXTRA = {
-    "ck_i8.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
+    "ck_i8.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1",
+                  "-mllvm", "-pragma-unroll-threshold=100000"],
 }
 
 

@@ -1055,6 +1055,9 @@ int ck_plan_ntt(ck_context *ctx, int n, int num_main, int num_ter, int num_aux,
   CK_REQUIRE(form >= 0 || !overlap, "autotuned plans need outputs that do not alias inputs");
   if (overlap) form = 0;
   const int limbs = num_main + num_ter + num_aux;
+  // large inverse transforms run in one pass on the int8 matrix cores
+  const bool inverse_one_pass =
+      inverse && !overlap && c.plan_ntt_form != 0 && one_pass_limbs((size_t)n * limbs) > 0;
   if (form != 0) {
     I8NttTabs T;
     const int rc = ntt8_tables(c, &T);
@@ -1067,6 +1070,8 @@ int ck_plan_ntt(ck_context *ctx, int n, int num_main, int num_ter, int num_aux,
     p->form = cd.form;
     int rc = kOk;
     if (cd.form == 0) {
+      p->one_pass = inverse_one_pass;
+      if (inverse_one_pass) p->form = 1;
       PlanSink sink(*p);
       for (int k = 0; k < n && !rc; k++) {
         sink.begin_item();
@@ -1097,11 +1102,14 @@ int ck_plan_ntt(ck_context *ctx, int n, int num_main, int num_ter, int num_aux,
     return rc;
   };
   std::vector<Plan::Candidate> cands;
+  const int total = n * limbs;
   if (form >= 0) {
-    cands.push_back({form, c.ntt8_blocks, c.ntt8_chunk, -1.0});
+    // one pass, unless the two-pass form's shape was chosen by option
+    const bool one_pass = one_pass_limbs(total) > 0 && c.ntt8_blocks == 16 && c.ntt8_chunk == 0;
+    cands.push_back({form, one_pass ? 0 : c.ntt8_blocks, c.ntt8_chunk, -1.0});
   } else {
     cands.push_back({0, 0, 0, -1.0});
-    const int total = n * limbs;
+    if (one_pass_limbs(total) > 0) cands.push_back({1, 0, 0, -1.0});
     for (int blocks : {16, 8, 4})
       for (int chunk : {0, 512, 256, 128})
         if (chunk == 0 || chunk < total) cands.push_back({1, blocks, chunk, -1.0});

@@ -25,6 +25,7 @@ struct I8NttTabs {
   const int32_t *planes = nullptr;  // [prime][kI8Ctx][4 planes][64 lanes][4]
   const int32_t *corr = nullptr;    // [prime][2][16] offset corrections
   const uint32_t *tw = nullptr;     // [prime] psi^(c (2 brv8(p) + 1)), 16 x 16 tiles
+  const int32_t *twm = nullptr;     // the same times 2^32, centred
 };
 
 // One limb of a batched int8 transform: dst = NTT(src) (x R when mont).
@@ -45,6 +46,45 @@ void launch_ntt8_cols(const Context &c, const I8NttTabs &T, const Ntt8Job *jobs,
                       int col_blocks, hipStream_t st);
 void launch_ntt8_rows(const Context &c, const I8NttTabs &T, const Ntt8Job *jobs, int n,
                       int row_blocks, hipStream_t st);
+
+// The same transform in one pass, a workgroup per limb: rounds of 256 limbs
+// (one per CU) of 38-41 us each however full. A batch of at least 192 limbs
+// takes it; of the limbs past its whole rounds, 128 and more too, fewer run
+// as two passes (7.5 us and 0.25 us a limb). Measured for 192 / 256 / 512 /
+// 2048 limbs, against two vector passes: forward 38 / 37 / 74 / 318 us against
+// 55 / 64 / 129 / 570, inverse 42 / 40 / 78 / 334 us against 52 / 62 / 120 /
+// 543; at 264 limbs a second round for 8 of them costs 63 and 70 us in all.
+constexpr int kOnePassLimbs = 192, kOnePassRound = 256, kOnePassTail = 128;
+inline size_t one_pass_limbs(size_t n) {  // how many of n limbs, the first ones
+  if (n < (size_t)kOnePassLimbs) return 0;
+  const size_t tail = n % kOnePassRound;
+  return n < (size_t)kOnePassRound || tail >= (size_t)kOnePassTail ? n : n - tail;
+}
+void launch_ntt1p_fwd(const Context &c, const I8NttTabs &T, const Ntt8Job *jobs, int n,
+                      hipStream_t st);
+
+// Device tables of the one-pass inverse transform (ntt1p_inv_tables).
+constexpr int kI8InvCtxRow = 1;   // + c0
+constexpr int kI8InvCtxCol = 17;  // + r0
+constexpr int kI8InvCtx = 33;
+struct I8InvTabs {
+  const int32_t *planes = nullptr;  // [prime][kI8InvCtx][4 planes][64 lanes][4]
+  const int32_t *corr = nullptr;    // [prime][16] offset corrections
+  const int32_t *twm = nullptr;     // [prime] inverse 4-step twiddles
+};
+// One limb: dst = INTT(src, or src (*) src2) c1 with c1m = c1 2^32 mod q
+// centred; canonical, or centred in [-(q - 1)/2, (q - 1)/2].
+struct Inv1pJob {
+  const uint32_t *src, *src2;
+  uint32_t *dst;
+  int32_t c1m;
+  int16_t prime, centred;
+};
+static_assert(sizeof(Inv1pJob) == 32, "Inv1pJob is one 32-byte record");
+int ntt1p_inv_tables(Context &c, I8InvTabs *out);
+// prod: every job has src2
+void launch_ntt1p_inv(const Context &c, const I8InvTabs &T, const Inv1pJob *jobs, int n,
+                      bool prod, hipStream_t st);
 
 // ---- BaseConv on the int8 matrix cores / on the vector unit ----------------
 

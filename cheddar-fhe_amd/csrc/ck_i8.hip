@@ -333,6 +333,372 @@ __global__ __launch_bounds__(256, 3) void ntt8_rows_kernel(const Ntt8Job *__rest
   }
 }
 
+// ---- one-pass transform -------------------------------------------------------
+
+// Exchange between the two 16-point stages of a pass: 16 blocks of 16 x 16
+// words, 20 words a row.
+constexpr int kXb = 324;
+// the same for 32 columns: blocks of 16 rows of 36 words
+constexpr int kXc = 16 * 36;
+
+// the modulus of a limb and the factor of fold_q
+struct FoldQ {
+  uint32_t q;
+  int qinv, c;
+};
+__device__ __forceinline__ FoldQ fold_consts(const PrimeTab &P, int pr) {
+  return FoldQ{P.q[pr], P.qinv[pr],
+               __builtin_amdgcn_readfirstlane(i8::fold_factor(P.qr[pr]))};
+}
+// a lane's four outputs of a tile mod q (|r| < 0.71 q)
+__device__ __forceinline__ void fold4(const Acc4 &A, const FoldQ &f, int r[4]) {
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+    r[i] = i8::fold_q(A.d[0][i], A.d[1][i], A.d[2][i], A.d[3][i], f.q, f.c);
+}
+__device__ __forceinline__ uint32_t canon_i(int r, uint32_t q) {  // |r| < q
+  const uint32_t u = (uint32_t)r, v = u + q;
+  return u < v ? u : v;
+}
+
+// Global access at a uniform base plus a 32-bit lane offset (scalar base
+// addressing: no 64-bit lane addresses to keep in registers).
+template <typename V>
+__device__ __forceinline__ V ld_at(const void *base, uint32_t off) {
+  typedef const __attribute__((address_space(1))) char gchar;
+  return *(const __attribute__((address_space(1))) V *)((gchar *)base + off);
+}
+__device__ __forceinline__ void st4_at(void *base, uint32_t off, v4u v) {
+  typedef __attribute__((address_space(1))) char gchar;
+  *(__attribute__((address_space(1))) v4u *)((gchar *)base + off) = v;
+}
+
+// Keeps the scheduler from moving global loads and stores across this point
+// (it sinks prefetches to their use to save registers).
+__device__ __forceinline__ void keep_loads() { __builtin_amdgcn_sched_barrier(0x38F); }
+
+// 4 x 4 transpose between the lane groups g = 0..3 and four registers: lane
+// group g of register h holds element (g, h) before and (h, g) after.
+__device__ __forceinline__ void swap_lanes(int &a, int &b, bool wide) {
+  typedef unsigned v2u __attribute__((ext_vector_type(2)));
+  const v2u r = wide ? __builtin_amdgcn_permlane32_swap((unsigned)a, (unsigned)b, false, false)
+                     : __builtin_amdgcn_permlane16_swap((unsigned)a, (unsigned)b, false, false);
+  a = (int)r[0];
+  b = (int)r[1];
+}
+__device__ __forceinline__ void transpose_groups(int &r0, int &r1, int &r2, int &r3) {
+  swap_lanes(r0, r2, true);
+  swap_lanes(r1, r3, true);
+  swap_lanes(r0, r1, false);
+  swap_lanes(r2, r3, false);
+}
+
+// Forward transform of a whole limb by one workgroup of 8 waves: the column
+// pass's output (128 packed words a lane) stays in registers. Wave w runs the
+// first stage of a pass for tiles 2w, 2w + 1 and the second stage for the same
+// pair, so that its second-stage matrices stay in registers and, in the column
+// pass, its results are rows 32w .. 32w + 31 whole: the row pass then needs one
+// 4 x 4 transpose between lane groups and no exchange of the limb.
+//
+// Column pass in blocks of 32 columns: a lane's 16-byte load holds the four
+// columns 4 cq + e of one row, which are the same vector n = (cq, r0 & 1) of
+// four tiles e. Software pipeline: between two barriers a wave runs the second
+// stage of one block (two in the row pass) and the first stage of the next;
+// blocks are loaded two ahead.
+//
+// Reads a limb and writes it once (the two-pass forms move it twice each way,
+// at 4.4 to 4.8 TB/s), about 48 vector instructions an element against 61
+// with FP64 recombination and 90 of the vector form. 2048 limbs: 470 -> 318
+// us. A limb takes a CU 38 us: two waves per SIMD (235 registers hold the
+// limb) keep the vector unit 55 % busy, the rest is waiting at barriers and
+// for memory (252 us with loads and stores out of the way). A loop over limbs
+// with the next one's loads issued early (256 registers, spills) took 350 us,
+// one column block per barrier 343 us, non-temporal stores 326 us.
+__global__ __launch_bounds__(512, 2) void ntt1p_fwd_kernel(const Ntt8Job *__restrict__ jobs,
+                                                           int njobs, I8NttTabs T, PrimeTab P) {
+  // two 32-column blocks of the column pass, four row blocks of the row pass
+  static_assert(4 * kXb >= 2 * kXc, "exchange size");
+  __shared__ __align__(16) int xs[4 * 16 * kXb];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int g = lane >> 4, n = lane & 15;
+  const v4i zero = {0, 0, 0, 0};
+  CJob &J = ((CJob *)jobs)[xcd_block(blockIdx.x, njobs)];
+  const int pr = J.prime, mont = J.mont;
+  const uint32_t *src = J.src;
+  uint32_t *dst = J.dst;
+  const FoldQ f = fold_consts(P, pr);
+  const uint32_t lane16 = 16 * lane;
+  const int32_t *pl = T.planes + (size_t)pr * kI8Ctx * 1024;
+  auto matrices = [&](int ca, int cb, v4i a[4], v4i b[2][4]) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) a[j] = ld_at<v4i>(pl + (ca * 4 + j) * 256, lane16);
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        b[k][j] = ld_at<v4i>(pl + ((cb + 2 * w + k) * 4 + j) * 256, lane16);
+  };
+  int Z[2][16][4];
+  {
+    // vector n = 2 cq + r0l: rows 2w + r0l + 16 (4 g + t), columns 4 cq + e
+    const int cq = n >> 1, r0l = n & 1;
+    const uint32_t in_off = 4 * ((64 * g + r0l) * 256 + 4 * cq);
+    v4u raw[2][4];
+    auto load = [&](int B) {
+#pragma unroll
+      for (int t = 0; t < 4; t++)
+        raw[B & 1][t] = ld_at<v4u>(src + (2 * w + 16 * t) * 256 + 32 * B, in_off);
+    };
+    load(0);
+    v4i a1[4], b1[2][4];
+    matrices(mont ? kI8CtxA1Mont : kI8CtxA1, kI8CtxB1, a1, b1);
+    const v4i corr = ld_at<v4i>(T.corr + (pr * 2 + mont) * 16, 16 * g);
+    load(1);
+    const int *tw0 = T.twm + (size_t)pr * kN + (size_t)(2 * w) * 4096;
+    v4i tw[2][2][2];
+    auto load_tw = [&](int B) {
+#pragma unroll
+      for (int c = 0; c < 2; c++)
+#pragma unroll
+        for (int k = 0; k < 2; k++)
+          tw[B & 1][c][k] = ld_at<v4i>(tw0 + (16 * k + 2 * B + c) * 256, lane16);
+    };
+    load_tw(0);
+    keep_loads();
+    auto stage1 = [&](int B) {
+      int r[4][4];
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const v4u *x = raw[B & 1];
+        const v4i b = {pack_off(x[0][e]), pack_off(x[1][e]), pack_off(x[2][e]),
+                       pack_off(x[3][e])};
+        fold4(mfma_tile(a1, b, corr), f, r[e]);
+      }
+      int *X = &xs[(B & 1) * 16 * kXc + 4 * g * kXc + (2 * w + r0l) * 36 + 4 * cq];
+#pragma unroll
+      for (int v = 0; v < 4; v++)
+        *(v4i *)(X + v * kXc) = v4i{pack_c(r[0][v]), pack_c(r[1][v]), pack_c(r[2][v]),
+                                    pack_c(r[3][v])};
+    };
+    stage1(0);
+    __syncthreads();
+#pragma unroll
+    for (int B = 0; B < 8; B++) {
+      if (B + 1 < 8) load_tw(B + 1);
+      if (B + 2 < 8) load(B + 2);
+      keep_loads();
+      if (B + 1 < 8) stage1(B + 1);
+#pragma unroll
+      for (int c = 0; c < 2; c++)
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+          const int *X = &xs[(B & 1) * 16 * kXc + (2 * w + k) * kXc + 4 * g * 36 + 16 * c + n];
+          const v4i bx = {X[0], X[36], X[72], X[108]};
+          int y[4];
+          fold4(mfma_tile(b1[k], bx, zero), f, y);
+#pragma unroll
+          for (int v = 0; v < 4; v++)
+            Z[k][2 * B + c][v] =
+                pack_c(i8::mont_centred(y[v], tw[B & 1][c][k][v], f.q, f.qinv));
+        }
+      __syncthreads();
+    }
+  }
+  v4i a3[4], b3[2][4];
+  matrices(kI8CtxA3, kI8CtxB3, a3, b3);
+  keep_loads();
+  // rows 16 (2w + k) + 4 g + v, columns 16 cb + n -> lane group = cb / 4
+#pragma unroll
+  for (int k = 0; k < 2; k++)
+#pragma unroll
+    for (int cl = 0; cl < 4; cl++)
+#pragma unroll
+      for (int v = 0; v < 4; v++)
+        transpose_groups(Z[k][cl][v], Z[k][4 + cl][v], Z[k][8 + cl][v], Z[k][12 + cl][v]);
+  auto stage3 = [&](int s) {  // rows 16 (2w + k) + s
+    const int h = s >> 2, v0 = s & 3;
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      const v4i b = {Z[k][4 * h][v0], Z[k][4 * h + 1][v0], Z[k][4 * h + 2][v0],
+                     Z[k][4 * h + 3][v0]};
+      int r[4];
+      fold4(mfma_tile(a3, b, zero), f, r);
+      int *W = &xs[(s & 3) * 16 * kXb + 4 * g * kXb + (2 * w + k) * 20 + n];
+#pragma unroll
+      for (int v = 0; v < 4; v++) W[v * kXb] = pack_c(r[v]);
+    }
+  };
+  stage3(0);
+  stage3(1);
+  __syncthreads();
+  // rows s + 16 n, columns 16 (2w + k) + 4 g + v: 16 bytes a lane
+  const uint32_t out_off = 4 * (16 * n * 256 + 4 * g);
+#pragma unroll
+  for (int s = 0; s < 16; s++) {
+    if (s + 2 < 16) stage3(s + 2);
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      const v4i bx = *(const v4i *)&xs[(s & 3) * 16 * kXb + (2 * w + k) * kXb + n * 20 + 4 * g];
+      int r[4];
+      fold4(mfma_tile(b3[k], bx, zero), f, r);
+      st4_at(dst + s * 256 + 32 * w + 16 * k, out_off,
+                v4u{canon_i(r[0], f.q), canon_i(r[1], f.q), canon_i(r[2], f.q),
+                    canon_i(r[3], f.q)});
+    }
+    if (s & 1) __syncthreads();
+  }
+}
+
+// Inverse transform of a whole limb, the mirror image: row pass (contract
+// q0, then q1), the inverse 4-step twiddle, the transpose between lane groups,
+// column pass (contract p0, then p1), then the limb's constant. 2048 limbs: 540
+// (two FP64 passes) -> 333 us, bound as the forward transform. Step s of the
+// row pass takes rows s + 16 n, vector n of every tile; step c1 of the column
+// pass columns 16 c1 .. 16 c1 + 15. PROD: the input is src (*) src2 (Montgomery).
+template <bool PROD>
+__global__ __launch_bounds__(512, 2) void ntt1p_inv_kernel(const Inv1pJob *__restrict__ jobs,
+                                                           int njobs, I8InvTabs T, PrimeTab P) {
+  __shared__ __align__(16) int xs[4 * 16 * kXb];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int g = lane >> 4, n = lane & 15;
+  const v4i zero = {0, 0, 0, 0};
+  typedef const __attribute__((address_space(4))) Inv1pJob CInv;
+  CInv &J = ((CInv *)jobs)[xcd_block(blockIdx.x, njobs)];
+  const int pr = J.prime;
+  const uint32_t *src = J.src, *src2 = J.src2;
+  uint32_t *dst = J.dst;
+  const FoldQ f = fold_consts(P, pr);
+  const uint32_t lane16 = 16 * lane;
+  const int32_t *pl = T.planes + (size_t)pr * kI8InvCtx * 1024;
+  // the common matrix, and the second-stage matrices 2w, 2w + 1 from context cb
+  v4i a[4], b[2][4];
+  auto second = [&](int cb) {
+#pragma unroll
+    for (int k = 0; k < 2; k++)
+#pragma unroll
+      for (int j = 0; j < 4; j++)
+        b[k][j] = ld_at<v4i>(pl + ((cb + 2 * w + k) * 4 + j) * 256, lane16);
+  };
+  int Z[2][16][4];
+  {
+    // row s + 16 n, columns 16 (2w + k) + 4 g + t
+    const uint32_t in_off = 4 * (16 * n * 256 + 4 * g);
+    constexpr int kAhead = PROD ? 3 : 4;
+    v4u raw[4][2], raw2[4][2];
+    auto load = [&](int s) {
+#pragma unroll
+      for (int k = 0; k < 2; k++) {
+        raw[s & 3][k] = ld_at<v4u>(src + s * 256 + 32 * w + 16 * k, in_off);
+        if (PROD) raw2[s & 3][k] = ld_at<v4u>(src2 + s * 256 + 32 * w + 16 * k, in_off);
+      }
+    };
+    const int *tw0 = T.twm + (size_t)pr * kN + (size_t)(2 * w) * 4096;
+    v4i tw[2][2];
+    auto load_tw = [&](int s) {
+#pragma unroll
+      for (int k = 0; k < 2; k++)
+        tw[s & 1][k] = ld_at<v4i>(tw0 + (16 * k + s) * 256, lane16);
+    };
+    load(0);
+    load(1);
+#pragma unroll
+    for (int j = 0; j < 4; j++) a[j] = ld_at<v4i>(pl + j * 256, lane16);
+    second(kI8InvCtxRow);
+    const v4i corr = ld_at<v4i>(T.corr + pr * 16, 16 * g);
+#pragma unroll
+    for (int s = 2; s < kAhead; s++) load(s);
+    load_tw(0);
+    keep_loads();
+    auto stage1 = [&](int s) {
+      int r[2][4];
+#pragma unroll
+      for (int k = 0; k < 2; k++) {
+        v4u x = raw[s & 3][k];
+        if (PROD)
+#pragma unroll
+          for (int t = 0; t < 4; t++)
+            x[t] = sum_reduce((uint64_t)x[t] * raw2[s & 3][k][t], f.q, f.qinv);
+        const v4i d = {pack_off(x[0]), pack_off(x[1]), pack_off(x[2]), pack_off(x[3])};
+        fold4(mfma_tile(a, d, corr), f, r[k]);
+      }
+      int *X = &xs[(s & 3) * 16 * kXb + 4 * g * kXb + n * 20 + 2 * w];
+#pragma unroll
+      for (int v = 0; v < 4; v++)
+        *(int2 *)(X + v * kXb) = make_int2(pack_c(r[0][v]), pack_c(r[1][v]));
+    };
+    stage1(0);
+    stage1(1);
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < 16; s++) {
+      if (s + 1 < 16) load_tw(s + 1);
+      if (s + kAhead < 16) load(s + kAhead);
+      keep_loads();
+      if (s + 2 < 16) stage1(s + 2);
+#pragma unroll
+      for (int k = 0; k < 2; k++) {
+        const v4i d = *(const v4i *)&xs[(s & 3) * 16 * kXb + (2 * w + k) * kXb + n * 20 + 4 * g];
+        int y[4];
+        fold4(mfma_tile(b[k], d, zero), f, y);
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+          Z[k][s][v] = pack_c(i8::mont_centred(y[v], tw[s & 1][k][v], f.q, f.qinv));
+      }
+      if (s & 1) __syncthreads();
+    }
+  }
+  second(kI8InvCtxCol);
+  keep_loads();
+  // columns 2w + k + 16 (4 g + v), rows s + 16 n -> lane group = s / 4
+#pragma unroll
+  for (int k = 0; k < 2; k++)
+#pragma unroll
+    for (int sl = 0; sl < 4; sl++)
+#pragma unroll
+      for (int v = 0; v < 4; v++)
+        transpose_groups(Z[k][sl][v], Z[k][4 + sl][v], Z[k][8 + sl][v], Z[k][12 + sl][v]);
+  auto stage3 = [&](int c1) {  // columns 16 c1 + 2w + k
+    const int h = c1 >> 2, v0 = c1 & 3;
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      const v4i d = {Z[k][4 * h][v0], Z[k][4 * h + 1][v0], Z[k][4 * h + 2][v0],
+                     Z[k][4 * h + 3][v0]};
+      int r[4];
+      fold4(mfma_tile(a, d, zero), f, r);
+      int *W = &xs[(c1 & 3) * 16 * kXb + 4 * g * kXb + (2 * w + k) * 20 + n];
+#pragma unroll
+      for (int v = 0; v < 4; v++) W[v * kXb] = pack_c(r[v]);
+    }
+  };
+  stage3(0);
+  stage3(1);
+  __syncthreads();
+  // rows 2w + k + 16 n, columns 16 c1 + 4 g + v: 16 bytes a lane
+  const uint32_t out_off = 4 * (16 * n * 256 + 4 * g);
+  const int c1m = J.c1m, centred = J.centred;
+  const uint32_t above = centred ? (f.q - 1) >> 1 : f.q - 1;
+#pragma unroll
+  for (int c1 = 0; c1 < 16; c1++) {
+    if (c1 + 2 < 16) stage3(c1 + 2);
+#pragma unroll
+    for (int k = 0; k < 2; k++) {
+      const v4i d = *(const v4i *)&xs[(c1 & 3) * 16 * kXb + (2 * w + k) * kXb + n * 20 + 4 * g];
+      int r[4];
+      fold4(mfma_tile_t(d, b[k]), f, r);
+      v4u o;
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const uint32_t u = canon_i(i8::mont_centred(r[v], c1m, f.q, f.qinv), f.q);
+        o[v] = u > above ? u - f.q : u;
+      }
+      st4_at(dst + (2 * w + k) * 256 + 16 * c1, out_off, o);
+    }
+    if (c1 & 1) __syncthreads();
+  }
+}
+
 // ---- BaseConv ---------------------------------------------------------------
 
 typedef const __attribute__((address_space(4))) BconvI8Inst CBInst;
@@ -642,13 +1008,14 @@ uint32_t brv_n(uint32_t x, int bits) {
 
 int ntt8_tables(Context &c, I8NttTabs *out) {
   if (c.i8_planes) {
-    *out = I8NttTabs{c.i8_planes, c.i8_corr, c.i8_tw};
+    *out = I8NttTabs{c.i8_planes, c.i8_corr, c.i8_tw, c.i8_twm};
     return kOk;
   }
   const int np = c.num_primes;
   std::vector<int32_t> planes((size_t)np * kI8Ctx * 1024);
   std::vector<int32_t> corr((size_t)np * 32);
   std::vector<uint32_t> tw((size_t)np * kN);
+  std::vector<int32_t> twm((size_t)np * kN);
   uint32_t T[16][16];
   for (int pi = 0; pi < np; pi++) {
     const uint32_t q = c.primes[pi];
@@ -696,7 +1063,9 @@ int ntt8_tables(Context &c, I8NttTabs *out) {
       const int p1 = p >> 4, p0 = p & 15;
       for (int col = 0; col < 256; col++) {
         const int cb = col >> 4, cn = col & 15;
-        tp[(16 * p1 + cb) * 256 + (16 * (p0 >> 2) + cn) * 4 + (p0 & 3)] = (uint32_t)x;
+        const int at = (16 * p1 + cb) * 256 + (16 * (p0 >> 2) + cn) * 4 + (p0 & 3);
+        tp[at] = (uint32_t)x;
+        twm[(size_t)pi * kN + at] = i8::centre_h(x * rmod, q);
         x = x * step % q;
       }
     }
@@ -711,14 +1080,82 @@ int ntt8_tables(Context &c, I8NttTabs *out) {
   };
   int32_t *dp = nullptr, *dc = nullptr;
   uint32_t *dt = nullptr;
+  int32_t *dm = nullptr;
   int rc = up(&dp, planes);
   if (!rc) rc = up(&dc, corr);
   if (!rc) rc = up(&dt, tw);
+  if (!rc) rc = up(&dm, twm);
   if (rc) return rc;
   c.i8_planes = dp;
   c.i8_corr = dc;
   c.i8_tw = dt;
-  *out = I8NttTabs{dp, dc, dt};
+  c.i8_twm = dm;
+  *out = I8NttTabs{dp, dc, dt, dm};
+  return kOk;
+}
+
+// Tables of the one-pass inverse transform: with omega = psi^512,
+//   context 0          A[c0][q0]  = omega^(-16 c0 brv4(q0)), both passes,
+//   kI8InvCtxRow + c0  [c1][q1]   = omega^(-(c0 + 16 c1) brv4(q1)),
+//   kI8InvCtxCol + r0  [r1][p1]   = psi^(-256 (r0 + 16 r1)(2 brv4(p1) + 1)),
+// twm: psi^(-c (2 brv8(p) + 1)) 2^32, centred, for column c = c0 + 16 (4 g + v)
+// and row p = s + 16 n at word ((16 c0 + s) 64 + 16 g + n) 4 + v.
+int ntt1p_inv_tables(Context &c, I8InvTabs *out) {
+  if (c.i8_inv_planes) {
+    *out = I8InvTabs{c.i8_inv_planes, c.i8_inv_corr, c.i8_inv_twm};
+    return kOk;
+  }
+  const int np = c.num_primes;
+  std::vector<int32_t> planes((size_t)np * kI8InvCtx * 1024), corr((size_t)np * 16);
+  std::vector<int32_t> twm((size_t)np * kN);
+  uint32_t M[16][16];
+  std::vector<uint32_t> pw(2 * kN);  // psi^-k
+  for (int pi = 0; pi < np; pi++) {
+    const uint32_t q = c.primes[pi], inv = h_invmod(c.psi[pi], q);
+    const uint32_t rmod = (uint32_t)((1ull << 32) % q);
+    pw[0] = 1;
+    for (int k = 1; k < 2 * kN; k++) pw[k] = (uint32_t)((uint64_t)pw[k - 1] * inv % q);
+    auto at = [&](uint64_t k) { return pw[k & (2 * kN - 1)]; };
+    int32_t *pp = planes.data() + (size_t)pi * kI8InvCtx * 1024;
+    for (int m = 0; m < 16; m++) {
+      uint64_t s = 0;
+      for (int k = 0; k < 16; k++) s += M[m][k] = at(8192ull * m * brv_n(k, 4));
+      corr[(size_t)pi * 16 + m] =
+          i8::centre_h((uint64_t)h_mulmod((uint32_t)(s % q), (1u << 30) % q, q), q);
+    }
+    i8::ctx_planes(M, q, pp);
+    for (int x = 0; x < 16; x++) {
+      for (int m = 0; m < 16; m++)
+        for (int k = 0; k < 16; k++) M[m][k] = at(512ull * (x + 16 * m) * brv_n(k, 4));
+      i8::ctx_planes(M, q, pp + (size_t)(kI8InvCtxRow + x) * 1024);
+      for (int m = 0; m < 16; m++)
+        for (int k = 0; k < 16; k++)
+          M[m][k] = at(256ull * (x + 16 * m) * (2 * brv_n(k, 4) + 1));
+      i8::ctx_planes(M, q, pp + (size_t)(kI8InvCtxCol + x) * 1024);
+    }
+    int32_t *tp = twm.data() + (size_t)pi * kN;
+    for (int col = 0; col < 256; col++)
+      for (int p = 0; p < 256; p++) {
+        const int c1 = col >> 4, word = ((16 * (col & 15) + (p & 15)) * 64 + 16 * (c1 >> 2) +
+                                         (p >> 4)) * 4 + (c1 & 3);
+        tp[word] = i8::centre_h((uint64_t)at((uint64_t)col * (2 * brv_n(p, 8) + 1)) * rmod, q);
+      }
+  }
+  const int32_t **dst[3] = {&c.i8_inv_planes, &c.i8_inv_corr, &c.i8_inv_twm};
+  const std::vector<int32_t> *src[3] = {&planes, &corr, &twm};
+  const int32_t *dev[3];
+  for (int i = 0; i < 3; i++) {
+    int32_t *d = nullptr;
+    int rc = check_hip(hipMalloc((void **)&d, src[i]->size() * 4), "hipMalloc(int8 tables)");
+    if (rc) return rc;
+    c.allocations.push_back(d);
+    rc = check_hip(hipMemcpy(d, src[i]->data(), src[i]->size() * 4, hipMemcpyHostToDevice),
+                   "hipMemcpy(int8 tables)");
+    if (rc) return rc;
+    dev[i] = d;
+  }
+  for (int i = 0; i < 3; i++) *dst[i] = dev[i];
+  *out = I8InvTabs{dev[0], dev[1], dev[2]};
   return kOk;
 }
 
@@ -736,6 +1173,24 @@ void launch_ntt8_rows(const Context &c, const I8NttTabs &T, const Ntt8Job *jobs,
   const int nwg = n * (16 / row_blocks);
   launch(c, "ntt8_rows", n, ntt8_rows_kernel, dim3(nwg), dim3(256), st, jobs, nwg,
          row_blocks, T, c.ptab);
+}
+
+void launch_ntt1p_fwd(const Context &c, const I8NttTabs &T, const Ntt8Job *jobs, int n,
+                      hipStream_t st) {
+  if (n <= 0) return;
+  launch(c, "ntt1p_fwd", n, ntt1p_fwd_kernel, dim3(n), dim3(512), st, jobs, n,
+         T, c.ptab);
+}
+
+void launch_ntt1p_inv(const Context &c, const I8InvTabs &T, const Inv1pJob *jobs, int n,
+                      bool prod, hipStream_t st) {
+  if (n <= 0) return;
+  if (prod)
+    launch(c, "ntt1p_inv+tensor", n, ntt1p_inv_kernel<true>, dim3(n), dim3(512), st, jobs, n, T,
+           c.ptab);
+  else
+    launch(c, "ntt1p_inv", n, ntt1p_inv_kernel<false>, dim3(n), dim3(512), st, jobs, n, T,
+           c.ptab);
 }
 
 void launch_bconv_i8_table(const Context &c, const BconvI8Inst *insts, int n, int dsts,

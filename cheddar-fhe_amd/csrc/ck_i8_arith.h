@@ -56,6 +56,34 @@ CK_HD double reduce_q(double v, double q, double qr) {
   return __builtin_fma(-k, q, v);
 }
 
+// The factor of fold_q for q: 2^48 / q rounded (q > 2^17).
+CK_HD int fold_factor(double qr) { return (int)__builtin_rint(281474976710656.0 * qr); }
+
+// v = hi 2^16 + lo of combine() mod q, in 32-bit integers (full-rate
+// multiplies on gfx950; FP64 conversions and products take more issue slots
+// and a lower clock): with s = hi + floor(lo / 2^16),
+// k = floor(s c / 2^32 + 1/2), c = 2^48 / q + d, |d| <= 1/2, differs from v / q
+// by at most 1/2 + 2^16 / q + |s| 2^-33. For planes of 64 products
+// (|s| < 2^28.1, also with an offset correction below 2^30 in d_0, which
+// enters lo) that is below 1/2 + 2^16 / q + 2^-4.8, so the result r = v - k q,
+// exact modulo 2^32, is v mod q with |r| < 0.71 q for every q > 2^18.5 (the
+// smallest prime that is 1 mod 2^17 is 393217).
+CK_HD int fold_q(int d0, int d1, int d2, int d3, uint32_t q, int c) {
+  const int lo = d0 + d1 * 256;
+  const int hi = d2 + d3 * 256;
+  const int s = hi + (lo >> 16);
+  const int k = (int)(((int64_t)s * c + (1ll << 31)) >> 32);
+  return (int)(((uint32_t)hi << 16) + (uint32_t)lo - (uint32_t)k * q);
+}
+
+// a w 2^-32 mod q for |a| < q and a centred w = x 2^32 mod q: |result| <
+// 3/4 q (a Montgomery product; qinv = q^-1 mod 2^32)
+CK_HD int mont_centred(int a, int w, uint32_t q, int qinv) {
+  const int64_t p = (int64_t)a * w;
+  const int t = (int)((uint32_t)p * (uint32_t)qinv);
+  return (int)(p >> 32) - (int)(((int64_t)t * (int32_t)q) >> 32);
+}
+
 // ---- host side: operand tables --------------------------------------------
 
 inline uint32_t powmod_h(uint32_t a, uint64_t e, uint32_t q) {

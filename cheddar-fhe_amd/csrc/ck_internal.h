@@ -148,6 +148,8 @@ struct Context {
   // int8 matrix-core transform tables (built on first use, ck_i8.hip)
   const int32_t *i8_planes = nullptr, *i8_corr = nullptr;
   const uint32_t *i8_tw = nullptr;
+  const int32_t *i8_twm = nullptr;
+  const int32_t *i8_inv_planes = nullptr, *i8_inv_corr = nullptr, *i8_inv_twm = nullptr;
 
   std::vector<LevelPlan> levels;
   // Key switching at level -1 (the ModSwitchHandler of level -1 with

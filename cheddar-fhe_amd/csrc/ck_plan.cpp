@@ -145,6 +145,33 @@ void order_by_prime(PlanStage &s) {
     });
 }
 
+// Splits an inverse step: the first one_pass_limbs of its jobs become a
+// one-pass step (appended to out; the limb's constant turns into a Montgomery
+// operand), the others stay.
+int one_pass_inverse(Plan &p, PlanStage &s, std::vector<PlanStage> &out) {
+  const size_t take = one_pass_limbs(s.jobs.size());
+  const bool prod = s.flags_any & kInttLoadProduct;
+  for (const LimbJob &j : s.jobs)
+    if (((j.flags & kInttLoadProduct) != 0) != prod) return kOk;  // mixed: two passes
+  if (take == 0) return kOk;
+  if (!p.i8inv.planes) {
+    const int rc = ntt1p_inv_tables(*const_cast<Context *>(p.ctx), &p.i8inv);
+    if (rc) return rc;
+  }
+  PlanStage o;
+  o.kind = PlanStage::kInv1p;
+  o.flags_any = s.flags_any;
+  for (size_t i = 0; i < take; i++) {
+    const LimbJob &j = s.jobs[i];
+    const uint32_t q = p.ctx->primes[j.prime];
+    o.i1.push_back(Inv1pJob{j.src, j.src2, j.dst, i8::centre_h(h_to_mont(j.c1, q), q),
+                            (int16_t)j.prime, (int16_t)((j.flags & kInttCentred) != 0)});
+  }
+  s.jobs.erase(s.jobs.begin(), s.jobs.begin() + take);
+  out.push_back(std::move(o));
+  return kOk;
+}
+
 }  // namespace
 
 int plan_finish(Plan &p, bool mismatch) {
@@ -152,8 +179,18 @@ int plan_finish(Plan &p, bool mismatch) {
     set_error("plan items do not share one step sequence");
     return kErrUnsupported;
   }
+  std::vector<PlanStage> stages;
   for (PlanStage &s : p.stages) {
     order_by_prime(s);
+    if (s.kind == PlanStage::kInv && p.one_pass) {
+      const int rc = one_pass_inverse(p, s, stages);
+      if (rc) return rc;
+      if (s.jobs.empty()) continue;
+    }
+    stages.push_back(std::move(s));
+  }
+  p.stages = std::move(stages);
+  for (PlanStage &s : p.stages) {
     if (s.ka.size() > 65535 || s.bs.size() > 65535 || s.bc.size() > 65535 ||
         s.bi.size() > 65535) {
       set_error("too many items in one plan step");
@@ -167,6 +204,7 @@ int plan_finish(Plan &p, bool mismatch) {
     if (!rc) rc = upload_vec(p, &s.d_n8, s.n8);
     if (!rc) rc = upload_vec(p, &s.d_bi, s.bi);
     if (!rc) rc = upload_vec(p, &s.d_bq, s.bq);
+    if (!rc) rc = upload_vec(p, &s.d_i1, s.i1);
     if (rc) return rc;
   }
   return kOk;
@@ -184,6 +222,29 @@ void plan_add_ntt8(Plan &p, std::vector<Ntt8Job> jobs, int blocks, int chunk) {
   std::stable_sort(jobs.begin(), jobs.end(),
                    [](const Ntt8Job &a, const Ntt8Job &b) { return a.prime < b.prime; });
   const size_t n = jobs.size();
+  if (blocks == 0) {
+    p.stages.emplace_back();
+    PlanStage &one = p.stages.back();
+    one.kind = PlanStage::kNtt1p;
+    const size_t take = one_pass_limbs(n);
+    one.n8.assign(jobs.begin(), jobs.begin() + take);
+    if (take == n) return;
+    PlanStage rest;  // a short last round: two vector passes
+    rest.kind = PlanStage::kFwd;
+    for (size_t i = take; i < n; i++) {
+      LimbJob J;
+      std::memset(&J, 0, sizeof(J));
+      J.src = jobs[i].src;
+      J.dst = jobs[i].dst;
+      J.prime = (uint16_t)jobs[i].prime;
+      J.c1 = jobs[i].mont ? h_to_mont(1, p.ctx->primes[J.prime]) : 1u;
+      J.flags = jobs[i].mont ? kNttPreMul : 0;
+      rest.flags_any |= J.flags;
+      rest.jobs.push_back(J);
+    }
+    p.stages.push_back(std::move(rest));
+    return;
+  }
   const size_t step = chunk > 0 ? (size_t)chunk : n;
   for (size_t b = 0; b < n; b += step) {
     const size_t e = std::min(n, b + step);
@@ -232,6 +293,13 @@ int plan_run(const Plan &p, hipStream_t st) {
         break;
       case PlanStage::kNtt8Rows:
         launch_ntt8_rows(c, p.i8, s.d_n8, (int)s.n8.size(), s.blocks, st);
+        break;
+      case PlanStage::kNtt1p:
+        launch_ntt1p_fwd(c, p.i8, s.d_n8, (int)s.n8.size(), st);
+        break;
+      case PlanStage::kInv1p:
+        launch_ntt1p_inv(c, p.i8inv, s.d_i1, (int)s.i1.size(),
+                         (s.flags_any & kInttLoadProduct) != 0, st);
         break;
       case PlanStage::kBconvI8:
       case PlanStage::kBconvValu: {

@@ -12,6 +12,7 @@ struct PlanStage {
   enum Kind {
     kFwd, kInv, kKeyAccum, kKeyRows, kBsFused, kBconv,
     kNtt8Cols, kNtt8Rows,   // int8 matrix-core transform passes
+    kNtt1p, kInv1p,         // int8 matrix-core transforms in one pass
     kBconvI8, kBconvValu,   // BaseConv on the int8 matrix cores / vector unit
     kBconvCols              // BaseConv fused with the forward column stages
   } kind = kFwd;
@@ -21,15 +22,17 @@ struct PlanStage {
   std::vector<BsFusedItem> bs;
   std::vector<EwJob> ew;
   std::vector<BconvInst> bc;
-  std::vector<Ntt8Job> n8;      // kNtt8Cols / kNtt8Rows
+  std::vector<Ntt8Job> n8;      // kNtt8Cols / kNtt8Rows / kNtt1p
   std::vector<BconvI8Inst> bi;  // kBconvI8 / kBconvValu
   std::vector<BcolsQuad> bq;    // kBconvCols
+  std::vector<Inv1pJob> i1;     // kInv1p
   int blocks = 16;              // int8 passes: 16-column / 16-row blocks per workgroup
   LimbJob *d_jobs = nullptr;
   BconvInst *d_bc = nullptr;
   Ntt8Job *d_n8 = nullptr;
   BconvI8Inst *d_bi = nullptr;
   BcolsQuad *d_bq = nullptr;
+  Inv1pJob *d_i1 = nullptr;
   KeyAccumItem *d_ka = nullptr;
   BsFusedItem *d_bs = nullptr;
   EwJob *d_ew = nullptr;
@@ -57,6 +60,8 @@ struct Plan {
   };
   std::vector<Candidate> tuning;
   I8NttTabs i8{};
+  I8InvTabs i8inv{};
+  bool one_pass = true;  // large inverse steps in one pass
 };
 
 // Records the ops of one item after another; begin_item() rewinds to the
@@ -99,7 +104,7 @@ int plan_finish(Plan &p, bool mismatch);
 // Appends the int8 forward transform of `jobs` to p: column pass then row
 // pass per chunk of `chunk` limbs (0: all jobs in one chunk), so a chunk's
 // intermediate can stay in the last-level cache between its two passes;
-// jobs are ordered by prime first.
+// jobs are ordered by prime first. blocks = 0: the one-pass form.
 void plan_add_ntt8(Plan &p, std::vector<Ntt8Job> jobs, int blocks, int chunk);
 // a constant int table the plan owns (freed by plan_destroy)
 int plan_upload_i64(Plan &p, int64_t **dst, const std::vector<int64_t> &v);

@@ -360,9 +360,9 @@ int ck_plan_bconv(ck_context *ctx, const int *src_primes, int n_src,
                   uint32_t *const *dst, ck_plan **out);
 /* dst[k] = ck_ntt (inverse = 0) or ck_intt (inverse = 1) of src[k], k < n,
  * all with one NP (NTTHandler::NTT / INTT over a batch): one launch per pass
- * across the batch. The int8 form's column pass writes a tiled intermediate
- * over dst, so a plan whose outputs overlap its inputs (in place) uses the
- * vector form. */
+ * across the batch. From 192 limbs the int8 form runs in one pass, both ways.
+ * Its two-pass form writes a tiled intermediate over dst, so a plan whose
+ * outputs overlap its inputs (in place) uses the vector form. */
 int ck_plan_ntt(ck_context *ctx, int n, int num_main, int num_ter, int num_aux,
                 int inverse, int montgomery_conversion, const uint32_t *const *src,
                 uint32_t *const *dst, ck_plan **out);
@@ -416,11 +416,14 @@ int ck_plan_destroy(ck_plan *plan);
  * 0: radix-16 FP64 butterflies on the vector unit (NTTPhase1 / NTTPhase2,
  * src/core/NTT.cu:231-454); 1 (default, measured faster): the 4-step
  * 256 x 256 transform as exact int8 matrix products (residues split into
- * four bytes, int32 accumulation, exact recombination); -1: autotune, i.e. build the vector
- * form and the int8 form for every (CK_OPT_NTT8_BLOCKS, CK_OPT_NTT8_CHUNK)
+ * four bytes, int32 accumulation, exact recombination), in one pass from 192
+ * limbs unless CK_OPT_NTT8_BLOCKS or CK_OPT_NTT8_CHUNK is set; -1: autotune,
+ * i.e. build the vector form, the one-pass int8 form (blocks 0) and the
+ * two-pass int8 form for every (CK_OPT_NTT8_BLOCKS, CK_OPT_NTT8_CHUNK)
  * candidate, time each and keep the fastest (ck_plan_tuning lists them;
- * outputs must not alias inputs). Inverse transforms always use the vector
- * form. Results are identical. */
+ * outputs must not alias inputs). Inverse transforms use the one-pass int8
+ * form from 192 limbs (unless 0 is set), else the vector form. Results are
+ * identical. */
 #define CK_OPT_PLAN_NTT_FORM 4
 /* CK_OPT_PLAN_BCONV_FORM: the form of ck_plan_bconv. 0: FP64 matrix cores
  * (16-bit table halves); 1 (default, measured faster): int8 matrix cores

@@ -252,6 +252,61 @@ static void test_worst_case() {
   if (v != (double)want) fail("worst case combine", want, (long long)v);
 }
 
+// fold_q over the planes of 64 digit products, with and without an offset
+// correction below 2^30 in d_0, at random and at the bounds: congruent to the
+// recombined value and below 0.71 q; mont_centred over |a| < q and centred w:
+// the Montgomery product, below 3/4 q; bconv_quad_planes: every word holds the
+// digits of its destination, source and plane.
+static void test_fold(uint32_t q) {
+  const int c = fold_factor(1.0 / (double)q);
+  const int64_t b = 1 << 20, r30 = 1 << 30;
+  for (int i = 0; i < 200000; i++) {
+    int64_t d[4];
+    for (int j = 0; j < 4; j++)
+      d[j] = i < 64 ? ((i >> j & 1) ? b : -b) : uniform(-b, b);
+    if (i & 1) d[0] += i < 64 ? (i & 32 ? r30 : -r30) : uniform(-r30, r30);
+    const int r = fold_q((int)d[0], (int)d[1], (int)d[2], (int)d[3], q, c);
+    const __int128 want = (__int128)d[0] + (d[1] * 256) + (((__int128)d[2] + d[3] * 256) << 16);
+    if (mod_q((__int128)r - want, q) != 0 || std::abs((double)r) >= 0.71 * q)
+      fail("fold_q", (long long)r, (long long)mod_q(want, q));
+  }
+  uint32_t inv = 1;
+  for (int i = 0; i < 5; i++) inv *= 2 - q * inv;  // q^-1 mod 2^32
+  const int64_t h = q / 2;
+  for (int i = 0; i < 100000; i++) {
+    const int a = (int)(i < 4 ? (i & 1 ? (int64_t)q - 1 : 1 - (int64_t)q)
+                              : uniform(1 - (int64_t)q, (int64_t)q - 1));
+    const int w = (int)(i < 4 ? (i & 2 ? h : -h) : uniform(-h, h));
+    const int z = mont_centred(a, w, q, (int)inv);
+    if (mod_q(((__int128)z << 32) - (__int128)a * w, q) != 0 ||
+        std::abs((double)z) >= 0.751 * q)
+      fail("mont_centred", a, w);
+  }
+}
+
+static void test_quads(int S, int D, const std::vector<uint32_t> &mods) {
+  std::vector<uint32_t> tab((size_t)S * D), dq(D);
+  for (int d = 0; d < D; d++) {
+    dq[d] = mods[d % mods.size()];
+    for (int s = 0; s < S; s++) tab[(size_t)d * S + s] = (uint32_t)uniform(0, dq[d] - 1);
+  }
+  const std::vector<int32_t> pl = bconv_quad_planes(tab, S, D, dq);
+  const int words = bconv_quad_words(S), per = bconv_quad_per(S), lw = S <= 8 ? 2 : 4;
+  if (pl.size() != (size_t)((D + 3) / 4) * words) fail("quad size", (long long)pl.size(), words);
+  for (int quad = 0; quad < (D + 3) / 4; quad++)
+    for (int at = 0; at < words; at++) {
+      const int t = at % lw, lane = at / lw % 64, ks = at / lw / 64;
+      const int d = 4 * quad + (lane & 15) / 4, j = lane & 3;
+      const int s = 4 * per * ks + per * (lane >> 4) + t;
+      uint32_t want = 0;
+      if (t < per && d < D && s < S)
+        for (int i = 0; i < 4; i++)
+          want |= digit_byte(centre_h((uint64_t)tab[(size_t)d * S + s] *
+                                          powmod_h(2, 8 * i, dq[d]), dq[d]), j) << (8 * i);
+      if ((uint32_t)pl[(size_t)quad * words + at] != want) fail("quad word", at, d);
+    }
+}
+
 int main() {
   // chain prime, bootparam_40 main and terminal primes, 2^31 - 1, small
   const uint32_t primes[] = {2147352577u, 2100953089u, 1196556289u, 30539777u,
@@ -261,10 +316,14 @@ int main() {
   for (uint32_t q : primes) {
     test_reduce(q);
     test_stages(q);
+    test_fold(q);
   }
   const std::vector<uint32_t> mods(std::begin(primes), std::end(primes));
   for (int S : {1, 2, 7, 8, 9, 12, 16, 17, 24})
-    for (int D : {1, 16, 17, 32, 64}) test_bconv(S, D, mods);
+    for (int D : {1, 16, 17, 32, 64}) {
+      test_bconv(S, D, mods);
+      test_quads(S, D, mods);
+    }
   test_worst_case();
   std::printf("OK: %d failure(s)\n", failures);
   return failures ? 1 : 0;

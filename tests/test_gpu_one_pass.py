@@ -1,0 +1,54 @@
+"""GPU parity of the one-pass int8 transforms at the edges of their rule:
+the smallest batch that takes them, whole rounds of 256 limbs, a short last
+round (two vector passes) and a long one, both directions, both Montgomery
+options, primes of 20 to 31 bits, the residues 0, q - 1, (q - 1) / 2 and
+(q + 1) / 2 in every limb. Whole numbers: every word equals the oracle's."""
+import numpy as np
+import pytest
+
+from conftest import SEED_BASE, load_params
+from gpu_util import assert_same, uniform
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+@pytest.mark.parametrize("params,np3,polys,launches",
+                         [("rns24_aux8.json", (24, 0, 8), 6, 1),
+                          ("rns24_aux8.json", (16, 0, 0), 16, 1),
+                          ("rns24_aux8.json", (1, 0, 0), 257, 3),
+                          ("rns24_aux8.json", (24, 0, 8), 12, 1),
+                          ("rns24_aux8.json", (17, 0, 0), 11, 2),
+                          ("bootparam_40.json", (43, 4, 12), 4, 1),
+                          ("bootparam_30.json", (48, 0, 12), 4, 1)])
+@pytest.mark.parametrize("inverse,mont", [(False, False), (False, True), (True, True),
+                                          (True, False)])
+def test_one_pass(params, np3, polys, launches, inverse, mont):
+    import cheddar_amd as ck
+    import ckks_oracle as O
+    d = load_params(params)
+    ctx, P = ck.Context.from_json(d), O.Param.from_json(d)
+    O.set_threads(8)
+    pidx = P.np_primes(*np3)
+    kinds = min(polys, 5)  # distinct polynomials, repeated over the batch
+    xs = []
+    for k in range(kinds):
+        x = uniform(P, pidx, SEED_BASE + 5500 + k)
+        for i, p in enumerate(pidx):
+            q = P.prime(p)
+            x[i, :4] = x[i, -4:] = (0, q - 1, (q - 1) // 2, (q + 1) // 2)
+        xs.append(x)
+    xs[-1][:] = np.array([P.prime(p) - 1 for p in pidx], np.uint32)[:, None]
+    fn = P.intt_np if inverse else P.ntt_np
+    want = [fn(x, *np3, mont_conv=mont) for x in xs]
+    src = [ck.to_device(xs[k % kinds]) for k in range(polys)]
+    dst = [torch.full_like(s, -1) for s in src]
+    plan = ck.Plan.ntt(ctx, src, dst, np3, inverse=inverse, mont_conv=mont)
+    limbs = polys * sum(np3)
+    # 187 limbs: below the rule, the two passes of either form
+    assert plan.info()["launches"] == launches, limbs
+    plan.run()
+    torch.cuda.synchronize()
+    for k in range(polys):
+        assert_same(ck.to_host(dst[k]), want[k % kinds], f"poly {k}")
