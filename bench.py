@@ -97,8 +97,9 @@ def measured_traffic(kernel):
 
 
 # ---- rocprofv3 output summaries --------------------------------------------
-# Launch grids -> limb counts: column passes run 8 workgroups per limb,
-# row passes and element-wise kernels 16 / 64 per limb (grid y = limbs).
+# Launch grids -> limb counts: column passes run 16 workgroups per limb with 16
+# values a thread, 32 or 64 with four (by their size, 512 or 256 threads); row
+# passes and element-wise kernels 64 per limb (grid y = limbs).
 def _short(sym):
     s = sym.replace("void ", "").replace("ck::(anonymous namespace)::", "")
     s = s.replace("ck::", "").split("(")[0]
@@ -106,7 +107,7 @@ def _short(sym):
     return s[:-7] if s.endswith("_kernel") else s
 
 
-_KERNELS = ("ntt_fwd_cols", "intt_cols", "ntt_fwd_rows", "intt_rows", "key_accum",
+_KERNELS = ("ntt_fwd_cols", "intt_cols", "ntt_fwd_cols4", "intt_cols4", "ntt_fwd_rows", "intt_rows", "key_accum",
             "key_accum_table", "bs_fused", "bs_fused_table", "tensor", "permute",
             "binary", "unary", "const", "accum", "imag_unit", "crt_lift", "bconv_mfma",
             "bconv_mfma_table", "key_rows", "key_rows_table", "gs_accum")
@@ -128,6 +129,8 @@ def _limbs(short, grid_x, grid_y, wg_x):
         return None
     if short in ("ntt_fwd_cols", "intt_cols"):
         return wgs // 16
+    if short in ("ntt_fwd_cols4", "intt_cols4"):
+        return wgs * wg_x // 16384
     if short in ("bs_fused", "bs_fused_table"):
         return wgs // 64
     return grid_y
@@ -180,8 +183,10 @@ def pmc_traffic(fetch_csv, write_csv, scale=None):
             grid = int(r["Grid_Size"])
             if short in ("ntt_fwd_cols", "intt_cols"):
                 n = grid // wg // 16
+            elif short in ("ntt_fwd_cols4", "intt_cols4"):
+                n = grid // 16384
             elif short in ("ntt_fwd_rows", "intt_rows", "key_rows"):
-                n = grid // wg // 16
+                n = grid // wg // 64
             elif short in ("key_accum", "tensor", "permute"):
                 n = grid // wg // 64
             elif short in ("gs_accum", "permute_accum"):

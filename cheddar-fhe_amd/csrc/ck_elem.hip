@@ -5,6 +5,7 @@
 // products of stored values exactly as the reference's MultMontgomery
 // (include/common/Basic.cuh:251-260), so outputs are bit-identical.
 #include "ck_elem.h"
+#include "ck_radix16.h"
 
 namespace ck {
 namespace {
@@ -525,10 +526,10 @@ __device__ __forceinline__ void bs_fused_row(const EwNp &np, const PrimeTab &P,
       rb[d & 255] = sum_reduce(sb[i], q, qinv);
       ra[d & 255] = sum_reduce(sa[i], q, qinv);
     }
-    __builtin_amdgcn_wave_barrier();  // one wave's LDS accesses run in order
+    wave_sync();
     const uint4 ob = *reinterpret_cast<const uint4 *>(rb + lane4);
     const uint4 oa = *reinterpret_cast<const uint4 *>(ra + lane4);
-    __builtin_amdgcn_wave_barrier();
+    wave_sync();
     const size_t o = (size_t)y * 65536 + (d & 0xFF00u) + lane4;
     st4(A.out_b[r] + o, ob);
     st4(A.out_a[r] + o, oa);

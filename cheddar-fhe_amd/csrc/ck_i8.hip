@@ -377,22 +377,6 @@ __device__ __forceinline__ void st4_at(void *base, uint32_t off, v4u v) {
 // (it sinks prefetches to their use to save registers).
 __device__ __forceinline__ void keep_loads() { __builtin_amdgcn_sched_barrier(0x38F); }
 
-// 4 x 4 transpose between the lane groups g = 0..3 and four registers: lane
-// group g of register h holds element (g, h) before and (h, g) after.
-__device__ __forceinline__ void swap_lanes(int &a, int &b, bool wide) {
-  typedef unsigned v2u __attribute__((ext_vector_type(2)));
-  const v2u r = wide ? __builtin_amdgcn_permlane32_swap((unsigned)a, (unsigned)b, false, false)
-                     : __builtin_amdgcn_permlane16_swap((unsigned)a, (unsigned)b, false, false);
-  a = (int)r[0];
-  b = (int)r[1];
-}
-__device__ __forceinline__ void transpose_groups(int &r0, int &r1, int &r2, int &r3) {
-  swap_lanes(r0, r2, true);
-  swap_lanes(r1, r3, true);
-  swap_lanes(r0, r1, false);
-  swap_lanes(r2, r3, false);
-}
-
 // Forward transform of a whole limb by one workgroup of 8 waves: the column
 // pass's output (128 packed words a lane) stays in registers. Wave w runs the
 // first stage of a pass for tiles 2w, 2w + 1 and the second stage for the same

@@ -10,25 +10,23 @@
 //
 // MI355X mapping. A limb of 2^16 u32 is a 256 x 256 matrix (row = 256
 // consecutive coefficients).
-//   * row kernels (forward stages 8..15, inverse stages 0..7): a 256-thread
-//     workgroup owns 16 consecutive rows = one contiguous 16 KiB block; the
-//     side a thread holds 16 consecutive words of moves with 16-byte
-//     accesses, the other side straight between registers and memory with
-//     4-byte accesses (64 contiguous bytes per row and instruction).
-//   * column kernels (forward stages 0..7, inverse 8..15): a 256-thread
-//     workgroup owns all 256 rows x 16 columns; every load and store is a
-//     64-byte row segment per 16 lanes, read and written straight from
-//     registers (32 KiB of LDS: four workgroups and more fit a CU).
-// Each thread runs two radix-16 register phases on 16 values; the hand-off
-// between the two phases keeps the lazy doubles in an LDS tile (row tiles
-// use an XOR swizzle so both phase layouts are free of bank conflicts).
-// Twiddles are read once per workgroup phase as u32
-// and issued before the data loads. Butterflies use the exact FP64 modular
+//   * row kernels (forward stages 8..15, inverse stages 0..7): a wave owns one
+//     row, four values a lane, without a barrier; the transformed side moves
+//     with 16-byte accesses, the other with 4-byte accesses over 256
+//     contiguous bytes.
+//   * column kernels (forward stages 0..7, inverse 8..15): a workgroup owns all
+//     256 rows of 4, 8 or 16 columns (four values a thread, or 16 at 16
+//     columns), read and written straight from registers.
+// A wave with 16 values a thread works 1.4 us by itself, and a transform of a
+// few limbs leaves most of the chip idle meanwhile; four values a thread make
+// four times the waves and a fraction of the time: one limb, both passes,
+// 7.3 -> 5.0 us forward, 7.7 -> 5.1 us inverse.
+// Register phases are radix 4 (or 16); between them the lazy doubles move over
+// lane transposes or padded LDS words. Twiddles are read as u32 and issued
+// before the data loads. Butterflies use the exact FP64 modular
 // product of ck_arith.h with lazy ranges (integer doubles below 2^40); the
 // intermediate between the two passes of a transform is stored as a lazy
 // int32 in (-0.75 q, 0.75 q) and only final outputs are made canonical.
-// Each thread writes a phase's results back to exactly the LDS words it read
-// for that phase, so only the hand-offs between threads need a barrier.
 #include "ck_elem.h"
 #include "ck_internal.h"
 #include "ck_radix16.h"
@@ -38,42 +36,11 @@ namespace {
 
 constexpr int kN = 65536;
 constexpr int kRowThreads = 256;
-constexpr int kRowTile = 16;                  // rows per row-kernel workgroup
-constexpr int kRowTiles = 256 / kRowTile;     // per limb
+constexpr int kRowTile = 4;                // rows per row-kernel workgroup
+constexpr int kRowTiles = 256 / kRowTile;  // per limb
 constexpr int kColThreads = 256;
-constexpr int kColTile = 16;                  // columns per column workgroup
-constexpr int kColTiles = 256 / kColTile;     // per limb
-
-// ct16 with the twiddles kept in LDS, slot i of this thread at
-// tws[i * kRowThreads + threadIdx.x] (conflict-free): for a loop that runs
-// several transforms with the same twiddles and cannot keep them, and their
-// FP64 forms, in registers.
-__device__ __forceinline__ void ct16_lds(double x[16], const uint32_t *tws,
-                                         double q, double qr) {
-#pragma unroll
-  for (int s = 0; s < 4; s++) {
-    const int half = 8 >> s;
-#pragma unroll
-    for (int blk = 0; blk < (1 << s); blk++) {
-      const double w = (double)tws[((1 << s) - 1 + blk) * 256 + threadIdx.x];
-#pragma unroll
-      for (int j = 0; j < half; j++) {
-        double &a = x[blk * 2 * half + j];
-        double &b = x[blk * 2 * half + j + half];
-        const double r = mulmod_fq(b, w, q, qr);
-        b = a - r;
-        a = a + r;
-      }
-    }
-  }
-}
-
-// Row-tile LDS index: row rl, in-row offset b, XOR swizzle of the low nibble
-// by the high nibble (both b = t + 16k and b = 16t + j patterns hit 16
-// distinct banks).
-__device__ __forceinline__ int rlds(int rl, int b) {
-  return rl * 256 + (b ^ ((b >> 4) & 15));
-}
+constexpr int kColTile = 16;               // columns of a 16-value workgroup
+constexpr int kColTiles = 256 / kColTile;  // per limb
 
 // Launch descriptors: every kernel asks its descriptor for the LimbJob of
 // limb y (uniform per workgroup). JobByValue unpacks the kernel-argument
@@ -117,25 +84,7 @@ struct JobTable {
   }
 };
 
-// Row tile element b = t16 + 16 k of row rl straight from / to global
-// memory: each load or store instruction covers 64 contiguous bytes of each
-// of the wave's four rows, and no LDS staging or barrier is needed.
-__device__ __forceinline__ void rows_load_p1(const uint32_t *tile, int rl, int t16,
-                                             double x[16]) {
-  typedef const __attribute__((address_space(1))) int32_t gint;
-  gint *g = (gint *)(tile + rl * 256 + t16);
-#pragma unroll
-  for (int k = 0; k < 16; k++) x[k] = (double)g[16 * k];
-}
-__device__ __forceinline__ void rows_store_p1(uint32_t *tile, int rl, int t16,
-                                              const int32_t v[16]) {
-  typedef __attribute__((address_space(1))) int32_t gint;
-  gint *g = (gint *)(tile + rl * 256 + t16);
-#pragma unroll
-  for (int k = 0; k < 16; k++) g[16 * k] = v[k];
-}
-
-// Column tile of a launch: 16 tiles of 16 columns per limb; workgroup i
+// Column tile of the 16-value kernels: 16 tiles of 16 columns per limb; workgroup i
 // runs on XCD i mod 8, and tiles 2x and 2x + 1 (which share 128-byte lines)
 // are placed on the same XCD so a line is fetched into one L2 only.
 struct ColTile {
@@ -153,8 +102,128 @@ __device__ __forceinline__ int32_t lazy_i32(double x, const ModF &m) {
 }
 
 // ---------------------------------------------------------------------------
-// Forward, column stages s = 0..7 -> lazy int32 intermediate
+// Column passes: stages 0..7 of the forward transform, 8..15 of the inverse
 // ---------------------------------------------------------------------------
+//
+// A workgroup of NC waves owns NC columns, four rows a thread; with 16 / NC
+// values of `extra` in a lane's low four bits, e = wave 16 / NC + extra runs
+// over 0..15. The lane groups a = lane / 16 hold the row bits next to the
+// four registers', so two of the three hand-offs between radix-4 phases are
+// lane transposes and one goes through LDS. With few limbs a launch lasts as
+// long as one wave, and this form's waves work a quarter as long; which NC is
+// taken, and when 16 values a thread, stands at fwd_passes.
+template <int NC>
+struct ColLane {
+  int y, c, e, a;  // limb slot, column, e, lane group
+  __device__ __forceinline__ ColLane() {
+    // workgroup i runs on XCD i mod 8: the tiles of a 128-byte line share one
+    constexpr int kShare = 32 / NC, kTiles = 256 / NC;
+    const int b = blockIdx.x, l = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    y = b / kTiles;
+    c = (((b & 7) * kShare) | ((b >> 3) & (kShare - 1))) * NC + l % NC;
+    e = wv * (16 / NC) + (l & 15) / NC;
+    a = l >> 4;
+  }
+};
+// LDS word of a row: one spare row after every 16 keeps both sides of the
+// hand-off on distinct banks
+template <int NC>
+__device__ __forceinline__ int col_word(int row, int lane) {
+  return (row + (row >> 4)) * NC + lane % NC;
+}
+
+template <class D, int NC>
+__global__ __launch_bounds__(64 * NC) void ntt_fwd_cols4(const D desc, const PrimeTab P,
+                                                         const uint32_t *__restrict__ tw) {
+  __shared__ double lds[272 * NC];
+  const ColLane<NC> L;
+  const LimbJob J = desc.job(L.y);
+  const double q = P.qd[J.prime], qr = P.qr[J.prime];
+  const ModF m{q, qr};
+  const uint32_t *__restrict__ w = tw + (size_t)J.prime * kN;
+  const int e = L.e, a = L.a, C = 4 * e + a;
+  const uint32_t t0[3] = {w[1], w[2], w[3]};
+  const uint32_t t1[3] = {w[4 + a], w[8 + 2 * a], w[9 + 2 * a]};
+  const uint32_t t2[3] = {w[16 + e], w[32 + 2 * e], w[33 + 2 * e]};
+  const uint32_t t3[3] = {w[64 + C], w[128 + 2 * C], w[129 + 2 * C]};
+  // canonical residues (< 2^31) or a lazy signed BaseConv output, as int32
+  const int32_t *__restrict__ g =
+      reinterpret_cast<const int32_t *>(J.src) + (16 * a + e) * 256 + L.c;
+  double x[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) x[i] = (double)g[i * 64 * 256];
+  if (J.flags & kNttPreMul) {
+    const double cv = (double)J.c1, cq = cv * qr;
+#pragma unroll
+    for (int i = 0; i < 4; i++) x[i] = mulmod_f(x[i], cv, cq, q);
+  }
+  ct4(x, t0[0], t0 + 1, q, qr);  // rows 64 i + 16 a + e
+  transpose_groups(x);
+  ct4(x, t1[0], t1 + 1, q, qr);  // rows 64 a + 16 i + e
+#pragma unroll
+  for (int i = 0; i < 4; i++) lds[col_word<NC>(64 * a + 16 * i + e, threadIdx.x & 63)] = x[i];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 4; i++) x[i] = lds[col_word<NC>(16 * e + 4 * i + a, threadIdx.x & 63)];
+  ct4(x, t2[0], t2 + 1, q, qr);  // rows 16 e + 4 i + a
+  transpose_groups(x);
+  ct4(x, t3[0], t3 + 1, q, qr);  // rows 16 e + 4 a + i
+  uint32_t *__restrict__ o = J.dst + (16 * e + 4 * a) * 256 + L.c;
+#pragma unroll
+  for (int i = 0; i < 4; i++) o[i * 256] = (uint32_t)lazy_i32(x[i], m);
+}
+
+template <class D, int NC>
+__global__ __launch_bounds__(64 * NC) void intt_cols4(const D desc, const PrimeTab P,
+                                                      const uint32_t *__restrict__ tw) {
+  __shared__ double lds[272 * NC];
+  const ColLane<NC> L;
+  const LimbJob J = desc.job(L.y);
+  const double q = P.qd[J.prime], qr = P.qr[J.prime];
+  const uint32_t *__restrict__ w = tw + (size_t)J.prime * kN;
+  const int e = L.e, a = L.a, C = 4 * e + a;
+  const uint32_t t0[3] = {w[128 + 2 * C], w[129 + 2 * C], w[64 + C]};
+  const uint32_t t1[3] = {w[32 + 2 * e], w[33 + 2 * e], w[16 + e]};
+  const uint32_t t2[3] = {w[8 + 2 * a], w[9 + 2 * a], w[4 + a]};
+  const uint32_t t3[3] = {w[2], w[3], w[1]};
+  // the pass-1 intermediate (in dst) is lazy signed int32
+  const int32_t *__restrict__ g =
+      reinterpret_cast<const int32_t *>(J.dst) + (16 * e + 4 * a) * 256 + L.c;
+  double x[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) x[i] = (double)g[i * 256];
+  gs4(x, t0, t0[2], q, qr);  // rows 16 e + 4 a + i
+  transpose_groups(x);
+  gs4(x, t1, t1[2], q, qr);  // rows 16 e + 4 i + a
+#pragma unroll
+  for (int i = 0; i < 4; i++) lds[col_word<NC>(16 * e + 4 * i + a, threadIdx.x & 63)] = x[i];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 4; i++) x[i] = lds[col_word<NC>(64 * a + 16 * i + e, threadIdx.x & 63)];
+  gs4(x, t2, t2[2], q, qr);  // rows 64 a + 16 i + e
+  transpose_groups(x);
+  gs4(x, t3, t3[2], q, qr);  // rows 64 i + 16 a + e
+  const double cv = (double)J.c1, cq = cv * qr;
+  // x * c1 lands in (-0.75 q, 0.75 q): canonical [0, q) (above: never,
+  // below 0: + q) or centred [-(q-1)/2, (q-1)/2] (one fix-up either side)
+  // (integer fix-ups on the exact int32 conversion)
+  const int32_t qi = (int32_t)P.q[J.prime];
+  const bool centred = (J.flags & kInttCentred) != 0;
+  const int32_t above = centred ? (qi - 1) >> 1 : qi - 1;
+  const int32_t below = centred ? -((qi - 1) >> 1) : 0;
+  uint32_t *__restrict__ o = J.dst + (16 * a + e) * 256 + L.c;
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    int32_t v = (int32_t)mulmod_f(x[i], cv, cq, q);
+    v = v > above ? v - qi : v;
+    v = v < below ? v + qi : v;
+    o[i * 64 * 256] = (uint32_t)v;
+  }
+}
+
+// Many limbs: 16 values a thread, two radix-16 phases with one hand-off and no
+// lane transposes. Bound by vector issue (FP64 butterflies): 129 limbs take
+// 21.0 us (67 MB, 3.2 TB/s) where the four-value form takes 23.3.
 template <class D>
 __global__ __launch_bounds__(kColThreads, 5) void ntt_fwd_cols(
     const D desc, const PrimeTab P, const uint32_t *__restrict__ tw) {
@@ -206,170 +275,6 @@ __global__ __launch_bounds__(kColThreads, 5) void ntt_fwd_cols(
     o[(rb * 16 + j) * 256] = (uint32_t)lazy_i32(x[j], m);
 }
 
-// ---------------------------------------------------------------------------
-// Forward, row stages s = 8..15 (+ optional ModDown epilogue)
-// ---------------------------------------------------------------------------
-template <class D>
-__global__ __launch_bounds__(kRowThreads, 5) void ntt_fwd_rows(
-    const D desc, const PrimeTab P, const uint32_t *__restrict__ tw) {
-  __shared__ double ldsd[kRowTile * 256];
-  const int y = blockIdx.y;
-  const LimbJob J = desc.job(y);
-  const double q = P.qd[J.prime], qr = P.qr[J.prime];
-  const ModF m{q, qr};
-  const uint32_t *__restrict__ w = tw + (size_t)J.prime * kN;
-  const int rl = threadIdx.x >> 4;
-  const int t16 = threadIdx.x & 15;
-  const int r = blockIdx.x * kRowTile + rl;  // row within the limb
-  const size_t tile = (size_t)blockIdx.x * kRowTile * 256;
-
-  // phase 1 twiddles psi_rev[2^(8+s) + r 2^s + blk], phase 2
-  // psi_rev[2^(12+s) + r 2^(4+s) + t16 2^s + blk]
-  uint32_t t1[15], t2[15];
-#pragma unroll
-  for (int s = 0; s < 4; s++)
-#pragma unroll
-    for (int blk = 0; blk < (1 << s); blk++) {
-      t1[(1 << s) - 1 + blk] = w[(256 << s) + (r << s) + blk];
-      t2[(1 << s) - 1 + blk] =
-          w[(4096 << s) + (r << (4 + s)) + (t16 << s) + blk];
-    }
-  // the pass-1 intermediate (in dst) is lazy signed int32
-  double x[16];
-  rows_load_p1(J.dst + tile, rl, t16, x);
-  // the ModDown epilogue's second operand, issued with the data loads so its
-  // latency overlaps the row stages. Unconditional, since a conditional form
-  // costs a spill here: without an epilogue every lane reads the same first
-  // 64 bytes of the limb (one cached line per wave), unused.
-  const bool has2 = (J.flags & kNttModDownEpilogue) && J.src2;
-  const uint4 *s2p = reinterpret_cast<const uint4 *>(
-      has2 ? J.src2 + (size_t)r * 256 + t16 * 16 : J.dst);
-  uint4 s2[4];
-#pragma unroll
-  for (int i = 0; i < 4; i++) s2[i] = s2p[i];
-  ct16(x, t1, q, qr);
-#pragma unroll
-  for (int k = 0; k < 16; k++) ldsd[rlds(rl, t16 + 16 * k)] = x[k];
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < 16; j++) x[j] = ldsd[rlds(rl, 16 * t16 + j)];
-  ct16(x, t2, q, qr);
-
-  // this thread now holds the 16 consecutive outputs b = 16 t16 + j of row r
-  uint32_t out[16];
-  if (J.flags & kNttModDownEpilogue) {
-    // NTTPhase2ForModDown (NTT.cu:456-601): out = (src2 * pad - y) * ip
-    const double ip = (double)J.c3, ipq = ip * qr;
-    double a2[16];
-    if (has2) {
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const uint4 u = s2[i];
-        a2[4 * i + 0] = (double)u.x;
-        a2[4 * i + 1] = (double)u.y;
-        a2[4 * i + 2] = (double)u.z;
-        a2[4 * i + 3] = (double)u.w;
-      }
-      if (J.flags & kNttEpiloguePad) {
-        const double pv = (double)J.c2, pq = pv * qr;
-#pragma unroll
-        for (int j = 0; j < 16; j++) a2[j] = mulmod_f(a2[j], pv, pq, q);
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < 16; j++) a2[j] = 0.0;
-    }
-#pragma unroll
-    for (int j = 0; j < 16; j++)
-      out[j] = canon_small(mulmod_f(a2[j] - x[j], ip, ipq, q), q);
-  } else {
-#pragma unroll
-    for (int j = 0; j < 16; j++) out[j] = canon_f(x[j], m);
-  }
-  uint4 *o4 = reinterpret_cast<uint4 *>(J.dst + (size_t)r * 256 + t16 * 16);
-#pragma unroll
-  for (int i = 0; i < 4; i++)
-    o4[i] = make_uint4(out[4 * i], out[4 * i + 1], out[4 * i + 2],
-                       out[4 * i + 3]);
-}
-
-// ---------------------------------------------------------------------------
-// Inverse, row stages u = 0..7 -> lazy int32 intermediate
-// ---------------------------------------------------------------------------
-template <class D>
-__global__ __launch_bounds__(kRowThreads, 5) void intt_rows(
-    const D desc, const PrimeTab P, const uint32_t *__restrict__ tw) {
-  __shared__ double ldsd[kRowTile * 256];
-  const int y = blockIdx.y;
-  const LimbJob J = desc.job(y);
-  const double q = P.qd[J.prime], qr = P.qr[J.prime];
-  const ModF m{q, qr};
-  const uint32_t *__restrict__ w = tw + (size_t)J.prime * kN;
-  const int rl = threadIdx.x >> 4;
-  const int t16 = threadIdx.x & 15;
-  const int r = blockIdx.x * kRowTile + rl;
-  const size_t tile = (size_t)blockIdx.x * kRowTile * 256;
-
-  // phase 1 psi_inv_rev[2^(15-u) + r 2^(7-u) + t16 2^(3-u) + blk],
-  // phase 2 psi_inv_rev[2^(11-u) + r 2^(3-u) + blk]
-  uint32_t t1[15], t2[15];
-#pragma unroll
-  for (int u = 0; u < 4; u++)
-#pragma unroll
-    for (int blk = 0; blk < (8 >> u); blk++) {
-      t1[16 - (16 >> u) + blk] =
-          w[(32768 >> u) + (r << (7 - u)) + (t16 << (3 - u)) + blk];
-      t2[16 - (16 >> u) + blk] = w[(2048 >> u) + (r << (3 - u)) + blk];
-    }
-  // phase 1 reads b = 16 t16 + j: 64 contiguous bytes per thread
-  double x[16];
-  {
-    const uint4 *s4 =
-        reinterpret_cast<const uint4 *>(J.src + (size_t)r * 256 + t16 * 16);
-    if (J.flags & kInttLoadProduct) {
-      // Tensor's a1 (*) a2 (ElementWise.cu:504-546) fused into the load
-      const uint32_t qu = P.q[J.prime];
-      const int32_t qinv = P.qinv[J.prime];
-      const uint4 *t4 = reinterpret_cast<const uint4 *>(
-          J.src2 + (size_t)r * 256 + t16 * 16);
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const uint4 u = s4[i], w2 = t4[i];
-        x[4 * i + 0] = (double)mont_mul(u.x, w2.x, qu, qinv);
-        x[4 * i + 1] = (double)mont_mul(u.y, w2.y, qu, qinv);
-        x[4 * i + 2] = (double)mont_mul(u.z, w2.z, qu, qinv);
-        x[4 * i + 3] = (double)mont_mul(u.w, w2.w, qu, qinv);
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const uint4 u = s4[i];
-        x[4 * i + 0] = (double)u.x;
-        x[4 * i + 1] = (double)u.y;
-        x[4 * i + 2] = (double)u.z;
-        x[4 * i + 3] = (double)u.w;
-      }
-    }
-  }
-  gs16(x, t1, q, qr);
-  // GS sums double every stage: from inputs below 2^31 they stay below 2^39
-  // over all eight stages, well inside mulmod_f's range, so the hand-off
-  // needs no reduction
-#pragma unroll
-  for (int j = 0; j < 16; j++) ldsd[rlds(rl, 16 * t16 + j)] = x[j];
-  __syncthreads();
-#pragma unroll
-  for (int k = 0; k < 16; k++) x[k] = ldsd[rlds(rl, t16 + 16 * k)];
-  gs16(x, t2, q, qr);
-  int32_t o[16];
-#pragma unroll
-  for (int k = 0; k < 16; k++) o[k] = lazy_i32(x[k], m);
-  rows_store_p1(J.dst + tile, rl, t16, o);
-}
-
-// ---------------------------------------------------------------------------
-// Inverse, column stages u = 8..15, then the per-limb constant
-// ---------------------------------------------------------------------------
 template <class D>
 __global__ __launch_bounds__(kColThreads, 5) void intt_cols(
     const D desc, const PrimeTab P, const uint32_t *__restrict__ tw) {
@@ -429,153 +334,237 @@ __global__ __launch_bounds__(kColThreads, 5) void intt_cols(
 }
 
 // ---------------------------------------------------------------------------
+// Row passes: stages 8..15 of the forward transform, 0..7 of the inverse
+// ---------------------------------------------------------------------------
+//
+// A wave owns a row, four values a lane: one hand-off between the radix-4
+// phases is a lane transpose, two go through the wave's own LDS words, and no
+// barrier is needed. Against 16 rows a workgroup and 16 values a thread, both
+// passes of a forward transform: 1 limb 7.3 -> 6.0 us, 24 limbs 14.6 -> 12.6,
+// 59 limbs 26.5 -> 23.4. Above about 500 limbs the two are equal forward (which
+// follows the fused BaseConv there) and 16 values a thread are 8 % better
+// inverse, but such batches take the one-pass int8 form.
+constexpr int kRowPad = 320;  // doubles of a row: 4 spare ones after every 16
+__device__ __forceinline__ int pad16(int j) { return j + 4 * (j >> 4); }
+
+// twiddles of a forward row: phase p's three in t[p]
+struct RowTw {
+  uint32_t t[4][3];
+};
+__device__ __forceinline__ RowTw row_twiddles(const uint32_t *w, int r, int l) {
+  const int A = l >> 4, B = l >> 2;
+  const uint32_t *w1 = w + 1024 + 4 * r + A, *w1b = w + 2048 + 8 * r + 2 * A;
+  const uint32_t *w2 = w + 4096 + 16 * r + B, *w2b = w + 8192 + 32 * r + 2 * B;
+  const uint32_t *w3 = w + 16384 + 64 * r + l, *w3b = w + 32768 + 128 * r + 2 * l;
+  return RowTw{{{w[256 + r], w[512 + 2 * r], w[513 + 2 * r]},
+                {w1[0], w1b[0], w1b[1]},
+                {w2[0], w2b[0], w2b[1]},
+                {w3[0], w3b[0], w3b[1]}}};
+}
+// elements 64 i + l of a row in, elements 4 l + i of its transform (lazy) out
+__device__ __forceinline__ void row_forward(double x[4], const RowTw &T, int l, double *X,
+                                            double q, double qr) {
+  const int A = l >> 4, B = l >> 2;
+  ct4(x, T.t[0][0], T.t[0] + 1, q, qr);
+  transpose_groups(x);  // elements 64 A + 16 i + (l & 15)
+  ct4(x, T.t[1][0], T.t[1] + 1, q, qr);
+  wave_sync();
+#pragma unroll
+  for (int i = 0; i < 4; i++) X[pad16(64 * A + 16 * i + (l & 15))] = x[i];
+  wave_sync();
+#pragma unroll
+  for (int i = 0; i < 4; i++) x[i] = X[pad16(16 * B + 4 * i + (l & 3))];
+  ct4(x, T.t[2][0], T.t[2] + 1, q, qr);
+  wave_sync();
+#pragma unroll
+  for (int i = 0; i < 4; i++) X[pad16(16 * B + 4 * i + (l & 3))] = x[i];
+  wave_sync();
+#pragma unroll
+  for (int i = 0; i < 4; i++) x[i] = X[pad16(4 * l) + i];
+  ct4(x, T.t[3][0], T.t[3] + 1, q, qr);
+}
+
+template <class D>
+__global__ __launch_bounds__(kRowThreads) void ntt_fwd_rows(const D desc, const PrimeTab P,
+                                                            const uint32_t *__restrict__ tw) {
+  __shared__ double rows[kRowTile][kRowPad];
+  const LimbJob J = desc.job(blockIdx.y);
+  const double q = P.qd[J.prime], qr = P.qr[J.prime];
+  const ModF m{q, qr};
+  const int l = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int r = blockIdx.x * kRowTile + wv;
+  const RowTw T = row_twiddles(tw + (size_t)J.prime * kN, r, l);
+  // the pass-1 intermediate (in dst) is lazy signed int32
+  const int32_t *g = reinterpret_cast<const int32_t *>(J.dst) + r * 256 + l;
+  double x[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) x[i] = (double)g[64 * i];
+  // the ModDown epilogue's second operand, issued with the data loads
+  const bool has2 = (J.flags & kNttModDownEpilogue) && J.src2;
+  uint4 s2 = make_uint4(0, 0, 0, 0);
+  if (has2) s2 = *reinterpret_cast<const uint4 *>(J.src2 + r * 256 + 4 * l);
+  row_forward(x, T, l, rows[wv], q, qr);
+  uint32_t out[4];
+  if (J.flags & kNttModDownEpilogue) {
+    // NTTPhase2ForModDown (NTT.cu:456-601): out = (src2 * pad - y) * ip
+    const double ip = (double)J.c3, ipq = ip * qr;
+    double a2[4] = {(double)s2.x, (double)s2.y, (double)s2.z, (double)s2.w};
+    if (J.flags & kNttEpiloguePad) {
+      const double pv = (double)J.c2, pq = pv * qr;
+#pragma unroll
+      for (int i = 0; i < 4; i++) a2[i] = mulmod_f(a2[i], pv, pq, q);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++)
+      out[i] = canon_small(mulmod_f(a2[i] - x[i], ip, ipq, q), q);
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; i++) out[i] = canon_f(x[i], m);
+  }
+  *reinterpret_cast<uint4 *>(J.dst + r * 256 + 4 * l) =
+      make_uint4(out[0], out[1], out[2], out[3]);
+}
+
+template <class D>
+__global__ __launch_bounds__(kRowThreads) void intt_rows(const D desc, const PrimeTab P,
+                                                         const uint32_t *__restrict__ tw) {
+  __shared__ double rows[kRowTile][kRowPad];
+  const LimbJob J = desc.job(blockIdx.y);
+  const double q = P.qd[J.prime], qr = P.qr[J.prime];
+  const ModF m{q, qr};
+  const uint32_t *__restrict__ w = tw + (size_t)J.prime * kN;
+  const int l = threadIdx.x & 63;
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int r = blockIdx.x * kRowTile + wv;
+  const int A = l >> 4, B = l >> 2;
+  const uint32_t *w0 = w + 32768 + 128 * r + 2 * l, *w0b = w + 16384 + 64 * r + l;
+  const uint32_t *w1 = w + 8192 + 32 * r + 2 * B, *w1b = w + 4096 + 16 * r + B;
+  const uint32_t *w2 = w + 2048 + 8 * r + 2 * A, *w2b = w + 1024 + 4 * r + A;
+  const uint32_t t0[3] = {w0[0], w0[1], w0b[0]};
+  const uint32_t t1[3] = {w1[0], w1[1], w1b[0]};
+  const uint32_t t2[3] = {w2[0], w2[1], w2b[0]};
+  const uint32_t t3[3] = {w[512 + 2 * r], w[513 + 2 * r], w[256 + r]};
+  const uint4 u = *reinterpret_cast<const uint4 *>(J.src + r * 256 + 4 * l);
+  uint32_t in[4] = {u.x, u.y, u.z, u.w};
+  if (J.flags & kInttLoadProduct) {
+    // Tensor's a1 (*) a2 (ElementWise.cu:504-546) fused into the load
+    const uint4 v = *reinterpret_cast<const uint4 *>(J.src2 + r * 256 + 4 * l);
+    const uint32_t V[4] = {v.x, v.y, v.z, v.w};
+    const uint32_t qu = P.q[J.prime];
+    const int32_t qinv = P.qinv[J.prime];
+#pragma unroll
+    for (int i = 0; i < 4; i++) in[i] = mont_mul(in[i], V[i], qu, qinv);
+  }
+  double x[4] = {(double)in[0], (double)in[1], (double)in[2], (double)in[3]};
+  double *X = rows[wv];
+  gs4(x, t0, t0[2], q, qr);
+#pragma unroll
+  for (int i = 0; i < 4; i++) X[pad16(4 * l) + i] = x[i];
+  wave_sync();
+#pragma unroll
+  for (int i = 0; i < 4; i++) x[i] = X[pad16(16 * B + 4 * i + (l & 3))];
+  gs4(x, t1, t1[2], q, qr);
+  wave_sync();
+#pragma unroll
+  for (int i = 0; i < 4; i++) X[pad16(16 * B + 4 * i + (l & 3))] = x[i];
+  wave_sync();
+#pragma unroll
+  for (int i = 0; i < 4; i++) x[i] = X[pad16(64 * A + 16 * i + (l & 15))];
+  gs4(x, t2, t2[2], q, qr);
+  transpose_groups(x);  // elements 64 i + l
+  gs4(x, t3, t3[2], q, qr);
+  int32_t *o = reinterpret_cast<int32_t *>(J.dst) + r * 256 + l;
+#pragma unroll
+  for (int i = 0; i < 4; i++) o[64 * i] = lazy_i32(x[i], m);
+}
+
+// ---------------------------------------------------------------------------
 // Forward row stages fused with the key inner product (MultKeyNoModDown,
 // src/core/Context.cpp:609-712: the ModUp's last NTT stages, then
 // ElementWise::PAccum / CAccum, src/core/ElementWise.cu:225-366)
 // ---------------------------------------------------------------------------
 //
-// One workgroup owns a 16-row tile of output limb y (prime p). For every
-// ModUp group g it takes limb y of that group's ModUp output straight from
-// the column pass (lazy int32 in `modup`), runs the row stages in registers
-// and multiplies the 16 values each thread holds by the key limbs, so the
-// ModUp output never goes back to memory in NTT form. A group's own limbs
-// are the ModUp source itself (x, or the Tensor product a1 (*) a2). The
-// row outputs are made canonical and the products summed in 64 bits
-// (sum_fold, sum_reduce), as Montgomery products of the stored data:
+// One wave owns a row of output limb y (prime p). For every ModUp group g it
+// takes limb y of that group's ModUp output straight from the column pass
+// (lazy int32 in `modup`), runs the row stages in registers and multiplies the
+// four values each lane holds by the key limbs, so the ModUp output never goes
+// back to memory in NTT form. A group's own limbs are the ModUp source itself
+// (x, or the Tensor product a1 (*) a2). The row outputs are made canonical and
+// the products summed in 64 bits (sum_fold, sum_reduce), as Montgomery
+// products of the stored data:
 //   acc_x[y] = R^-1 (sum_g m_g * key_x,g + P R * fold_x)  mod q,
 // fold_b = d0 = b1 (*) b2 (HMult) or add_b, fold_a likewise, which is exactly
 // the key_accum kernel's sum.
 //
 // Bound by memory: the keys, 50 MB for 32 limbs and three groups, pass by
-// once, 111 MB in all at least. With every product reduced by itself in FP64
-// the kernel issued about 2540 vector instructions where it now has 1690:
-// 32 limbs 26.8 -> 23.4 us, 382 limbs of a batch 218 -> 195 us.
+// once, 111 MB in all at least. Products reduced one by one in FP64 -> sums in
+// 64 bits -> four values a lane instead of 16: 11 limbs 8.6 -> 6.8 us (last step), 32 limbs 26.8 -> 23.4 ->
+// 22.8, 59 limbs 47 -> 42, 382 limbs of a batch 218 -> 195 -> 164.
 template <class Args>
 __device__ __forceinline__ void key_rows_body(const EwNp &np, const PrimeTab &P,
                                               Args &A, const uint32_t *tw, int y,
-                                              double *ldsd, uint32_t *tws) {
+                                              double *X, int wv) {
   const int p = y < np.num_q ? np.q_prime0 + y : np.aux_prime0 + (y - np.num_q);
   const double q = P.qd[p], qr = P.qr[p];
   const ModF m{q, qr};
   const uint32_t qu = P.q[p];
   const int32_t qinv = P.qinv[p];
-  const uint32_t *__restrict__ w = tw + (size_t)p * kN;
-  const int rl = threadIdx.x >> 4;
-  const int t16 = threadIdx.x & 15;
-  const int r = blockIdx.x * kRowTile + rl;
-  const size_t tile = (size_t)blockIdx.x * kRowTile * 256;
+  const int l = threadIdx.x & 63;
+  const int r = blockIdx.x * kRowTile + wv;
   const size_t tot_stride = (size_t)np.num_total * kN;
-  const size_t off = (size_t)r * 256 + t16 * 16;  // this thread's 16 outputs
+  const uint32_t off = r * 256 + 4 * l;  // this thread's 4 outputs
   const size_t my = (size_t)y * kN + off;
   const int kl = y < np.num_q ? A.key_q0 + y : A.key_aux0 + (y - np.num_q);
   const size_t kp = (size_t)kl * kN + off;
   const bool tens = A.use_tensor && y < np.num_q;
+  const RowTw T = row_twiddles(tw + (size_t)p * kN, r, l);
 
-  // row-stage twiddles (as ntt_fwd_rows), parked in LDS for the group loop:
-  // slot i of this thread at tws[i * 256 + tid] (phase 1: 0..14, 2: 15..29);
-  // only this thread reads its slots back
-#pragma unroll
-  for (int s = 0; s < 4; s++)
-#pragma unroll
-    for (int blk = 0; blk < (1 << s); blk++) {
-      tws[((1 << s) - 1 + blk) * kRowThreads + threadIdx.x] = w[(256 << s) + (r << s) + blk];
-      tws[(15 + (1 << s) - 1 + blk) * kRowThreads + threadIdx.x] =
-          w[(4096 << s) + (r << (4 + s)) + (t16 << s) + blk];
-    }
-
-  uint64_t sb[16], sa[16];
-#pragma unroll
-  for (int j = 0; j < 16; j++) sb[j] = sa[j] = 0;
-  // the column-pass tile of the next group that needs the row stages is
-  // loaded one group ahead (into `pre`), so its latency overlaps the
-  // current group's arithmetic
-  auto next_rows_group = [&](int from) {
-    for (int i = from; i < A.ngroups; i++) {
-      const int g = A.group[i];
-      if (!(y >= A.own0[g] && y < A.own1[g])) return i;
-    }
-    return -1;
-  };
-  typedef const __attribute__((address_space(1))) int32_t gint;
-  int32_t pre[16];
-  auto prefetch = [&](int gi) {
-    gint *src = (gint *)(A.modup + (size_t)A.group[gi] * tot_stride + (size_t)y * kN + tile +
-                         rl * 256 + t16);
-#pragma unroll
-    for (int k = 0; k < 16; k++) pre[k] = src[16 * k];
-  };
-  int pg = next_rows_group(0);
-  if (pg >= 0) prefetch(pg);
+  uint64_t sb[4] = {0, 0, 0, 0}, sa[4] = {0, 0, 0, 0};
   for (int gi = 0; gi < A.ngroups; gi++) {
     const int g = A.group[gi];
     const bool own = (y >= A.own0[g] && y < A.own1[g]);
     // key limbs first: their loads overlap the row stages
-    uint4 kb[4], ka[4];
-    const uint32_t *kbp = A.key_b[g] + kp, *kap = A.key_a[g] + kp;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-      kb[i] = reinterpret_cast<const uint4 *>(kbp)[i];
-      ka[i] = reinterpret_cast<const uint4 *>(kap)[i];
-    }
-    uint32_t v[16];
+    const uint4 kb = *reinterpret_cast<const uint4 *>(A.key_b[g] + kp);
+    const uint4 ka = *reinterpret_cast<const uint4 *>(A.key_a[g] + kp);
+    uint32_t v[4];
     if (own) {
       if (tens) {
         // d2 = a1 (*) a2
-        const uint4 *a1 = reinterpret_cast<const uint4 *>(A.tensor[1] + my);
-        const uint4 *a2 = reinterpret_cast<const uint4 *>(A.tensor[3] + my);
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const uint4 u = a1[i], w2 = a2[i];
-          v[4 * i + 0] = sum_reduce((uint64_t)u.x * w2.x, qu, qinv);
-          v[4 * i + 1] = sum_reduce((uint64_t)u.y * w2.y, qu, qinv);
-          v[4 * i + 2] = sum_reduce((uint64_t)u.z * w2.z, qu, qinv);
-          v[4 * i + 3] = sum_reduce((uint64_t)u.w * w2.w, qu, qinv);
-        }
+        const uint4 a1 = *reinterpret_cast<const uint4 *>(A.tensor[1] + my);
+        const uint4 a2 = *reinterpret_cast<const uint4 *>(A.tensor[3] + my);
+        v[0] = sum_reduce((uint64_t)a1.x * a2.x, qu, qinv);
+        v[1] = sum_reduce((uint64_t)a1.y * a2.y, qu, qinv);
+        v[2] = sum_reduce((uint64_t)a1.z * a2.z, qu, qinv);
+        v[3] = sum_reduce((uint64_t)a1.w * a2.w, qu, qinv);
       } else {
-        const uint4 *xs = reinterpret_cast<const uint4 *>(A.x + my);
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const uint4 u = xs[i];
-          v[4 * i + 0] = u.x;
-          v[4 * i + 1] = u.y;
-          v[4 * i + 2] = u.z;
-          v[4 * i + 3] = u.w;
-        }
+        const uint4 u = *reinterpret_cast<const uint4 *>(A.x + my);
+        v[0] = u.x;
+        v[1] = u.y;
+        v[2] = u.z;
+        v[3] = u.w;
       }
     } else {
-      // gi == pg: its tile is in `pre`; start the next one
-      double x[16];
+      const int32_t *src = reinterpret_cast<const int32_t *>(
+          A.modup + (size_t)g * tot_stride + (size_t)y * kN + r * 256 + l);
+      double x[4];
 #pragma unroll
-      for (int k = 0; k < 16; k++) x[k] = (double)pre[k];
-      pg = next_rows_group(gi + 1);
-      if (pg >= 0) prefetch(pg);
-      ct16_lds(x, tws, q, qr);
-      __syncthreads();  // the previous group's exchange may still be read
+      for (int i = 0; i < 4; i++) x[i] = (double)src[64 * i];
+      row_forward(x, T, l, X, q, qr);
 #pragma unroll
-      for (int k = 0; k < 16; k++) ldsd[rlds(rl, t16 + 16 * k)] = x[k];
-      __syncthreads();
-#pragma unroll
-      for (int j = 0; j < 16; j++) x[j] = ldsd[rlds(rl, 16 * t16 + j)];
-      ct16_lds(x, tws + 15 * kRowThreads, q, qr);
-#pragma unroll
-      for (int j = 0; j < 16; j++) v[j] = canon_f(x[j], m);
+      for (int i = 0; i < 4; i++) v[i] = canon_f(x[i], m);
     }
-    const bool fold = gi & 1;  // two products between folds
+    const uint32_t KB[4] = {kb.x, kb.y, kb.z, kb.w}, KA[4] = {ka.x, ka.y, ka.z, ka.w};
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      const uint32_t KB[4] = {kb[i].x, kb[i].y, kb[i].z, kb[i].w};
-      const uint32_t KA[4] = {ka[i].x, ka[i].y, ka[i].z, ka[i].w};
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        sb[4 * i + e] += (uint64_t)v[4 * i + e] * KB[e];
-        sa[4 * i + e] += (uint64_t)v[4 * i + e] * KA[e];
-      }
+      sb[i] += (uint64_t)v[i] * KB[i];
+      sa[i] += (uint64_t)v[i] * KA[i];
     }
-    if (fold) {
+    if (gi & 1) {  // two products between folds
 #pragma unroll
-      for (int j = 0; j < 16; j++) {
-        sb[j] = sum_fold(sb[j], qu);
-        sa[j] = sum_fold(sa[j], qu);
+      for (int i = 0; i < 4; i++) {
+        sb[i] = sum_fold(sb[i], qu);
+        sa[i] = sum_fold(sa[i], qu);
       }
     }
   }
@@ -583,76 +572,64 @@ __device__ __forceinline__ void key_rows_body(const EwNp &np, const PrimeTab &P,
   // the P fold on q limbs: one more product (at most two since a fold)
   const uint32_t pp = y < np.num_q ? A.p_prod[p] : 0u;
   if (tens) {
-    const uint4 *b1 = reinterpret_cast<const uint4 *>(A.tensor[0] + my);
-    const uint4 *a1 = reinterpret_cast<const uint4 *>(A.tensor[1] + my);
-    const uint4 *b2 = reinterpret_cast<const uint4 *>(A.tensor[2] + my);
-    const uint4 *a2 = reinterpret_cast<const uint4 *>(A.tensor[3] + my);
+    const uint4 u1 = *reinterpret_cast<const uint4 *>(A.tensor[0] + my);
+    const uint4 v1 = *reinterpret_cast<const uint4 *>(A.tensor[1] + my);
+    const uint4 u2 = *reinterpret_cast<const uint4 *>(A.tensor[2] + my);
+    const uint4 v2 = *reinterpret_cast<const uint4 *>(A.tensor[3] + my);
+    const uint32_t B1[4] = {u1.x, u1.y, u1.z, u1.w}, A1[4] = {v1.x, v1.y, v1.z, v1.w};
+    const uint32_t B2[4] = {u2.x, u2.y, u2.z, u2.w}, A2[4] = {v2.x, v2.y, v2.z, v2.w};
 #pragma unroll
     for (int i = 0; i < 4; i++) {
-      const uint4 u1 = b1[i], v1 = a1[i], u2 = b2[i], v2 = a2[i];
-      const uint32_t B1[4] = {u1.x, u1.y, u1.z, u1.w}, A1[4] = {v1.x, v1.y, v1.z, v1.w};
-      const uint32_t B2[4] = {u2.x, u2.y, u2.z, u2.w}, A2[4] = {v2.x, v2.y, v2.z, v2.w};
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        const uint32_t d0 = sum_reduce((uint64_t)B1[e] * B2[e], qu, qinv);
-        const uint32_t d1 =
-            sum_reduce((uint64_t)B1[e] * A2[e] + (uint64_t)A1[e] * B2[e], qu, qinv);
-        sb[4 * i + e] += (uint64_t)pp * d0;
-        sa[4 * i + e] += (uint64_t)pp * d1;
-      }
+      const uint32_t d0 = sum_reduce((uint64_t)B1[i] * B2[i], qu, qinv);
+      const uint32_t d1 =
+          sum_reduce((uint64_t)B1[i] * A2[i] + (uint64_t)A1[i] * B2[i], qu, qinv);
+      sb[i] += (uint64_t)pp * d0;
+      sa[i] += (uint64_t)pp * d1;
     }
   } else if (y < np.num_q && (A.add_b || A.add_a)) {
+    if (A.add_b) {
+      const uint4 u = *reinterpret_cast<const uint4 *>(A.add_b + my);
+      const uint32_t U[4] = {u.x, u.y, u.z, u.w};
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-      if (A.add_b) {
-        const uint4 u = reinterpret_cast<const uint4 *>(A.add_b + my)[i];
-        const uint32_t U[4] = {u.x, u.y, u.z, u.w};
+      for (int i = 0; i < 4; i++) sb[i] += (uint64_t)pp * U[i];
+    }
+    if (A.add_a) {
+      const uint4 u = *reinterpret_cast<const uint4 *>(A.add_a + my);
+      const uint32_t U[4] = {u.x, u.y, u.z, u.w};
 #pragma unroll
-        for (int e = 0; e < 4; e++) sb[4 * i + e] += (uint64_t)pp * U[e];
-      }
-      if (A.add_a) {
-        const uint4 u = reinterpret_cast<const uint4 *>(A.add_a + my)[i];
-        const uint32_t U[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-        for (int e = 0; e < 4; e++) sa[4 * i + e] += (uint64_t)pp * U[e];
-      }
+      for (int i = 0; i < 4; i++) sa[i] += (uint64_t)pp * U[i];
     }
   }
 
-  uint4 *ob = reinterpret_cast<uint4 *>(A.out_b + my);
-  uint4 *oa = reinterpret_cast<uint4 *>(A.out_a + my);
+  uint32_t vb[4], va[4];
 #pragma unroll
   for (int i = 0; i < 4; i++) {
-    uint32_t vb[4], va[4];
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-      vb[e] = sum_reduce(sum_fold(sb[4 * i + e], qu), qu, qinv);
-      va[e] = sum_reduce(sum_fold(sa[4 * i + e], qu), qu, qinv);
-    }
-    ob[i] = make_uint4(vb[0], vb[1], vb[2], vb[3]);
-    oa[i] = make_uint4(va[0], va[1], va[2], va[3]);
+    vb[i] = sum_reduce(sum_fold(sb[i], qu), qu, qinv);
+    va[i] = sum_reduce(sum_fold(sa[i], qu), qu, qinv);
   }
+  *reinterpret_cast<uint4 *>(A.out_b + my) = make_uint4(vb[0], vb[1], vb[2], vb[3]);
+  *reinterpret_cast<uint4 *>(A.out_a + my) = make_uint4(va[0], va[1], va[2], va[3]);
 }
 
-__global__ __launch_bounds__(kRowThreads, 2) void key_rows_kernel(
+__global__ __launch_bounds__(kRowThreads) void key_rows_kernel(
     const EwNp np, const PrimeTab P, const KeyAccumArgs A, const uint32_t *__restrict__ tw) {
-  __shared__ double ldsd[kRowTile * 256];
-  __shared__ uint32_t tws[30 * kRowThreads];
-  key_rows_body(np, P, A, tw, blockIdx.y, ldsd, tws);
+  __shared__ double rows[kRowTile][kRowPad];
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  key_rows_body(np, P, A, tw, blockIdx.y, rows[wv], wv);
 }
 
-__global__ __launch_bounds__(kRowThreads, 2) void key_rows_table_kernel(
+__global__ __launch_bounds__(kRowThreads) void key_rows_table_kernel(
     const KeyAccumItem *__restrict__ items, const EwJob *__restrict__ jobs,
     const PrimeTab P, const uint32_t *__restrict__ tw) {
-  __shared__ double ldsd[kRowTile * 256];
-  __shared__ uint32_t tws[30 * kRowThreads];
+  __shared__ double rows[kRowTile][kRowPad];
+  const int wv = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   typedef const __attribute__((address_space(4))) KeyAccumItem CItem;
   typedef const __attribute__((address_space(4))) EwJob CJob;
   CJob &jb = ((CJob *)jobs)[blockIdx.y];
   const int item = jb.item, y = jb.y;
   CItem &it = ((CItem *)items)[item];
   const EwNp np{it.np.num_q, it.np.num_total, it.np.q_prime0, it.np.aux_prime0};
-  key_rows_body(np, P, it.A, tw, y, ldsd, tws);
+  key_rows_body(np, P, it.A, tw, y, rows[wv], wv);
 }
 
 const char *fwd_rows_name(int flags) {
@@ -662,23 +639,49 @@ const char *inv_rows_name(int flags) {
   return (flags & kInttLoadProduct) ? "intt_rows+tensor" : "intt_rows";
 }
 
+// Column pass over n limbs. A small launch lasts as long as one wave, so few
+// limbs take four values a thread over four (n <= 4) or eight columns a
+// workgroup, more than 64 the 16-value form. Both passes of a forward transform
+// with four columns / eight columns / 16 values, us: 1 limb 5.0 / 5.3 / 6.0,
+// 4 limbs 5.7 / 5.8 / 6.6, 8 limbs 7.1 / 6.9 / 7.6, 24 limbs 12.8 / 12.4 / 12.6,
+// 59 limbs 24.0 / 23.3 / 23.4; inverse 1 limb 5.1 / 5.4 / 6.4, 24 limbs 13.2 /
+// 12.6 / 13.3, 59 limbs 24.1 / 22.8 / 22.5.
+constexpr int kCols4 = 4, kCols8 = 64;
+
 template <class D>
 void fwd_passes(const Context &ctx, const D &d, int n, int flags, hipStream_t st) {
-  if (!(flags & kNttRowsOnly))
-    launch(ctx, "ntt_fwd_cols", n, ntt_fwd_cols<D>, dim3(kColTiles * n), dim3(kColThreads),
-           st, d, ctx.ptab, (const uint32_t *)ctx.d_tw_fwd);
+  const uint32_t *tw = ctx.d_tw_fwd;
+  if (!(flags & kNttRowsOnly)) {
+    auto cols = [&](auto kernel, int wgs, int threads) {
+      launch(ctx, "ntt_fwd_cols", n, kernel, dim3(wgs * n), dim3(threads), st, d, ctx.ptab, tw);
+    };
+    if (n <= kCols4)
+      cols(ntt_fwd_cols4<D, 4>, 64, 256);
+    else if (n <= kCols8)
+      cols(ntt_fwd_cols4<D, 8>, 32, 512);
+    else
+      cols(ntt_fwd_cols<D>, kColTiles, kColThreads);
+  }
   if (!(flags & kNttColsOnly))
     launch(ctx, fwd_rows_name(flags), n, ntt_fwd_rows<D>, dim3(kRowTiles, n),
-           dim3(kRowThreads), st, d, ctx.ptab, (const uint32_t *)ctx.d_tw_fwd);
+           dim3(kRowThreads), st, d, ctx.ptab, tw);
 }
 
 template <class D>
 void inv_passes(const Context &ctx, const D &d, int n, int flags,
                 hipStream_t st) {
-  launch(ctx, inv_rows_name(flags), n, intt_rows<D>, dim3(kRowTiles, n),
-         dim3(kRowThreads), st, d, ctx.ptab, (const uint32_t *)ctx.d_tw_inv);
-  launch(ctx, "intt_cols", n, intt_cols<D>, dim3(kColTiles * n),
-         dim3(kColThreads), st, d, ctx.ptab, (const uint32_t *)ctx.d_tw_inv);
+  const uint32_t *tw = ctx.d_tw_inv;
+  launch(ctx, inv_rows_name(flags), n, intt_rows<D>, dim3(kRowTiles, n), dim3(kRowThreads), st,
+         d, ctx.ptab, tw);
+  auto cols = [&](auto kernel, int wgs, int threads) {
+    launch(ctx, "intt_cols", n, kernel, dim3(wgs * n), dim3(threads), st, d, ctx.ptab, tw);
+  };
+  if (n <= kCols4)
+    cols(intt_cols4<D, 4>, 64, 256);
+  else if (n <= kCols8)
+    cols(intt_cols4<D, 8>, 32, 512);
+  else
+    cols(intt_cols<D>, kColTiles, kColThreads);
 }
 
 }  // namespace

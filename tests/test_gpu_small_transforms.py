@@ -1,0 +1,61 @@
+"""GPU parity of the two-pass transforms at the edges of the column kernels'
+rule: four columns a workgroup (to 4 limbs), eight (to 64), 16 values a thread
+above; single calls and plans, both directions, in place and not, primes of 20
+to 31 bits, the residues 0, q - 1, (q - 1) / 2 and (q + 1) / 2 in every limb.
+Whole numbers: every word equals the oracle's."""
+import pytest
+
+from conftest import SEED_BASE, load_params
+from gpu_util import assert_same, uniform
+
+pytestmark = pytest.mark.gpu
+
+torch = pytest.importorskip("torch")
+
+
+def _inputs(P, pidx, count):
+    xs = []
+    for k in range(count):
+        x = uniform(P, pidx, SEED_BASE + 6100 + k)
+        for i, p in enumerate(pidx):
+            q = P.prime(p)
+            x[i, :4] = x[i, -4:] = (0, q - 1, (q - 1) // 2, (q + 1) // 2)
+            x[i, 256:512] = q - 1
+        xs.append(x)
+    return xs
+
+
+@pytest.mark.parametrize("inverse", [False, True])
+@pytest.mark.parametrize("params,np3,polys",
+                         [("rns24_aux8.json", (1, 0, 0), 1),
+                          ("bootparam_40.json", (1, 1, 2), 1),
+                          ("bootparam_30.json", (3, 0, 2), 1),
+                          ("rns24_aux8.json", (24, 0, 8), 1),
+                          ("bootparam_40.json", (43, 4, 12), 1),
+                          ("rns24_aux8.json", (1, 0, 0), 4),
+                          ("bootparam_30.json", (5, 0, 0), 1),
+                          ("rns24_aux8.json", (24, 0, 8), 2),
+                          ("rns24_aux8.json", (5, 0, 8), 5)])
+def test_small_transform(params, np3, polys, inverse):
+    import cheddar_amd as ck
+    import ckks_oracle as O
+    d = load_params(params)
+    ctx, P = ck.Context.from_json(d), O.Param.from_json(d)
+    O.set_threads(8)
+    xs = _inputs(P, P.np_primes(*np3), polys)
+    fn = P.intt_np if inverse else P.ntt_np
+    want = [fn(x, *np3, mont_conv=inverse) for x in xs]
+    src = [ck.to_device(x) for x in xs]
+    dst = [torch.full_like(s, -1) for s in src]
+    ck.Plan.ntt(ctx, src, dst, np3, inverse=inverse, mont_conv=inverse).run()
+    torch.cuda.synchronize()
+    for k in range(polys):
+        assert_same(ck.to_host(dst[k]), want[k], f"plan, poly {k}")
+    call = ctx.intt if inverse else ctx.ntt
+    for k in range(polys):
+        call(dst[k], src[k], *np3, mont_conv=inverse)
+        call(src[k], src[k], *np3, mont_conv=inverse)
+    torch.cuda.synchronize()
+    for k in range(polys):
+        assert_same(ck.to_host(dst[k]), want[k], f"call, poly {k}")
+        assert_same(ck.to_host(src[k]), want[k], f"call in place, poly {k}")
