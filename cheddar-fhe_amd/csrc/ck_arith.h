@@ -8,9 +8,12 @@
 //   * exact FP64 modular products for transforms: a residue is held as a
 //     double (integers up to 2^53 are exact), a * w mod q is computed as
 //     hi = a*w, lo = fma(a, w, -hi) (the exact rounding error), k =
-//     rint(a * w/q), r = fma(-k, q, hi) + lo. FP64 FMA is full rate on
-//     CDNA4 while 32-bit integer multiplies are quarter rate, so transforms
-//     use this form. Both families produce the same canonical residues.
+//     rint(a * w/q), r = fma(-k, q, hi) + lo. FP64 and 32-bit integer
+//     multiplies issue at about the same rate on gfx950 (5.4 and 4.7 cycles a
+//     wave), and a butterfly is 8 FP64 instructions against about 10 integer
+//     ones, so the vector transforms use this form; sums of products, one
+//     64-bit multiply-add each, are integer (below). Both families produce the
+//     same canonical residues.
 #pragma once
 
 #include <hip/hip_runtime.h>

@@ -176,9 +176,10 @@ __global__ __launch_bounds__(kThreads) void accum_kernel(const EwNp np,
 // operand and is masked to zero afterwards), so the loads of a giant step
 // are all in flight before its first product.
 //
-// Arithmetic in exact FP64 instead of 32-bit Montgomery products (whose
-// multiplies issue at a quarter of the FP64 rate): with the plaintext word
-// split as m = mh 2^14 + ml, the sums Sh = sum x mh (< 16 2^31 2^17 = 2^52)
+// Bound by memory over its many operands (59 limbs, 8 baby and 8 giant steps:
+// 325 us, 4.6 TB/s), not by arithmetic: 64-bit integer sums take 331 us there
+// and, with 16 baby steps, 453 us against 331. In exact FP64, with the
+// plaintext word split as m = mh 2^14 + ml, the sums Sh = sum x mh (< 16 2^31 2^17 = 2^52)
 // and Sl = sum x ml (< 2^49) over at most 16 terms are exact doubles, and
 //   sum_t x_t (*) m_t = R^-1 (Sh 2^14 + Sl)  mod q
 // is one reduction of Sh 2^14 (a power-of-two scaling, exact), one FP64
