@@ -373,10 +373,6 @@ __device__ __forceinline__ void st4_at(void *base, uint32_t off, v4u v) {
   *(__attribute__((address_space(1))) v4u *)((gchar *)base + off) = v;
 }
 
-// Keeps the scheduler from moving global loads and stores across this point
-// (it sinks prefetches to their use to save registers).
-__device__ __forceinline__ void keep_loads() { __builtin_amdgcn_sched_barrier(0x38F); }
-
 // Forward transform of a whole limb by one workgroup of 8 waves: the column
 // pass's output (128 packed words a lane) stays in registers. Wave w runs the
 // first stage of a pass for tiles 2w, 2w + 1 and the second stage for the same

@@ -58,6 +58,10 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Keeps the scheduler from moving global loads and stores across this point
+// (it sinks prefetches to their use to save registers).
+__device__ __forceinline__ void keep_loads() { __builtin_amdgcn_sched_barrier(0x38F); }
+
 // 4 x 4 transpose between the lane groups g = 0..3 and four registers: lane
 // group g of register h holds element (g, h) before and (h, g) after.
 __device__ __forceinline__ void swap_lanes(int &a, int &b, bool wide) {
