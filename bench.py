@@ -99,7 +99,8 @@ def measured_traffic(kernel):
 # ---- rocprofv3 output summaries --------------------------------------------
 # Launch grids -> limb counts: column passes run 16 workgroups per limb with 16
 # values a thread, 32 or 64 with four (by their size, 512 or 256 threads); row
-# passes and element-wise kernels 64 per limb (grid y = limbs).
+# passes 64 per limb or, with 16 values a thread, 16 (grid y = limbs),
+# element-wise kernels 64.
 def _short(sym):
     s = sym.replace("void ", "").replace("ck::(anonymous namespace)::", "")
     s = s.replace("ck::", "").split("(")[0]
@@ -107,10 +108,11 @@ def _short(sym):
     return s[:-7] if s.endswith("_kernel") else s
 
 
-_KERNELS = ("ntt_fwd_cols", "intt_cols", "ntt_fwd_cols4", "intt_cols4", "ntt_fwd_rows", "intt_rows", "key_accum",
-            "key_accum_table", "bs_fused", "bs_fused_table", "tensor", "permute",
-            "binary", "unary", "const", "accum", "imag_unit", "crt_lift", "bconv_mfma",
-            "bconv_mfma_table", "key_rows", "key_rows_table", "gs_accum")
+_KERNELS = ("ntt_fwd_cols", "intt_cols", "ntt_fwd_cols4", "intt_cols4", "ntt_fwd_rows",
+            "intt_rows", "ntt_fwd_rows16", "intt_rows16", "key_accum", "key_accum_table",
+            "bs_fused", "bs_fused_table", "tensor", "permute", "binary", "unary", "const",
+            "accum", "imag_unit", "crt_lift", "bconv_mfma", "bconv_mfma_table", "key_rows",
+            "key_rows_table", "gs_accum")
 # int8 matrix-core kernels (batched plans): labelled by workgroup count, since
 # their workgroups per limb depend on the plan's blocks per workgroup
 _I8_KERNELS = ("ntt8_cols", "ntt8_rows", "ntt1p_fwd", "ntt1p_inv", "bconv_i8", "bconv_valu",
@@ -187,6 +189,8 @@ def pmc_traffic(fetch_csv, write_csv, scale=None):
                 n = grid // 16384
             elif short in ("ntt_fwd_rows", "intt_rows", "key_rows"):
                 n = grid // wg // 64
+            elif short in ("ntt_fwd_rows16", "intt_rows16"):
+                n = grid // wg // 16
             elif short in ("key_accum", "tensor", "permute"):
                 n = grid // wg // 64
             elif short in ("gs_accum", "permute_accum"):

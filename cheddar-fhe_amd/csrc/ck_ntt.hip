@@ -38,6 +38,8 @@ constexpr int kN = 65536;
 constexpr int kRowThreads = 256;
 constexpr int kRowTile = 4;                // rows per row-kernel workgroup
 constexpr int kRowTiles = 256 / kRowTile;  // per limb
+constexpr int kRow16Tile = 16;             // rows of a 16-value workgroup
+constexpr int kRow16Tiles = 256 / kRow16Tile;
 constexpr int kColThreads = 256;
 constexpr int kColTile = 16;               // columns of a 16-value workgroup
 constexpr int kColTiles = 256 / kColTile;  // per limb
@@ -348,9 +350,7 @@ __global__ __launch_bounds__(kColThreads, 5) void intt_cols(
 // phases is a lane transpose, two go through the wave's own LDS words, and no
 // barrier is needed. Against 16 rows a workgroup and 16 values a thread, both
 // passes of a forward transform: 1 limb 7.3 -> 6.0 us, 24 limbs 14.6 -> 12.6,
-// 59 limbs 26.5 -> 23.4. Above about 500 limbs the two are equal forward (which
-// follows the fused BaseConv there) and 16 values a thread are 8 % better
-// inverse, but such batches take the one-pass int8 form.
+// 59 limbs 26.5 -> 23.4. Many limbs take the 16-value kernels below.
 constexpr int kRowPad = 320;  // doubles of a row: 4 spare ones after every 16
 __device__ __forceinline__ int pad16(int j) { return j + 4 * (j >> 4); }
 
@@ -484,6 +484,103 @@ __global__ __launch_bounds__(kRowThreads) void intt_rows(const D desc, const Pri
   int32_t *o = reinterpret_cast<int32_t *>(J.dst) + r * 256 + l;
 #pragma unroll
   for (int i = 0; i < 4; i++) o[64 * i] = lazy_i32(x[i], m);
+}
+
+// Many limbs: 16 values a thread, 16 rows a workgroup (a contiguous 16 KiB), two
+// radix-16 phases with one hand-off. Bound by memory and FP64 issue together:
+// 2048 limbs inverse 244 us (4.4 TB/s) where four values a lane take 286,
+// forward 257 against 285. The lines between the two stand at fwd_passes.
+//
+// Row-tile LDS index: row rl, in-row offset b, the low nibble swizzled by the
+// high nibble (b = t + 16 k and b = 16 t + j both hit 16 distinct banks).
+__device__ __forceinline__ int row16_word(int rl, int b) {
+  return rl * 256 + (b ^ ((b >> 4) & 15));
+}
+
+// no ModDown epilogue
+template <class D>
+__global__ __launch_bounds__(kRowThreads, 5) void ntt_fwd_rows16(
+    const D desc, const PrimeTab P, const uint32_t *__restrict__ tw) {
+  __shared__ double lds[kRow16Tile * 256];
+  const LimbJob J = desc.job(blockIdx.y);
+  const double q = P.qd[J.prime], qr = P.qr[J.prime];
+  const ModF m{q, qr};
+  const uint32_t *__restrict__ w = tw + (size_t)J.prime * kN;
+  const int rl = threadIdx.x >> 4, t = threadIdx.x & 15;
+  const int r = blockIdx.x * kRow16Tile + rl;
+  // phase 1 twiddles psi_rev[2^(8+s) + r 2^s + blk], phase 2
+  // psi_rev[2^(12+s) + r 2^(4+s) + t 2^s + blk]
+  uint32_t t1[15], t2[15];
+#pragma unroll
+  for (int s = 0; s < 4; s++)
+#pragma unroll
+    for (int blk = 0; blk < (1 << s); blk++) {
+      t1[(1 << s) - 1 + blk] = w[(256 << s) + (r << s) + blk];
+      t2[(1 << s) - 1 + blk] = w[(4096 << s) + (r << (4 + s)) + (t << s) + blk];
+    }
+  // the pass-1 intermediate (in dst) is lazy signed int32; elements t + 16 k
+  const int32_t *g = reinterpret_cast<const int32_t *>(J.dst) + r * 256 + t;
+  double x[16];
+#pragma unroll
+  for (int k = 0; k < 16; k++) x[k] = (double)g[16 * k];
+  ct16(x, t1, q, qr);
+#pragma unroll
+  for (int k = 0; k < 16; k++) lds[row16_word(rl, t + 16 * k)] = x[k];
+  __syncthreads();
+#pragma unroll
+  for (int j = 0; j < 16; j++) x[j] = lds[row16_word(rl, 16 * t + j)];
+  ct16(x, t2, q, qr);
+  uint4 *o = reinterpret_cast<uint4 *>(J.dst + r * 256 + 16 * t);
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+    o[i] = make_uint4(canon_f(x[4 * i], m), canon_f(x[4 * i + 1], m),
+                      canon_f(x[4 * i + 2], m), canon_f(x[4 * i + 3], m));
+}
+
+// no product input
+template <class D>
+__global__ __launch_bounds__(kRowThreads, 5) void intt_rows16(
+    const D desc, const PrimeTab P, const uint32_t *__restrict__ tw) {
+  __shared__ double lds[kRow16Tile * 256];
+  const LimbJob J = desc.job(blockIdx.y);
+  const double q = P.qd[J.prime], qr = P.qr[J.prime];
+  const ModF m{q, qr};
+  const uint32_t *__restrict__ w = tw + (size_t)J.prime * kN;
+  const int rl = threadIdx.x >> 4, t = threadIdx.x & 15;
+  const int r = blockIdx.x * kRow16Tile + rl;
+  // phase 1 psi_inv_rev[2^(15-u) + r 2^(7-u) + t 2^(3-u) + blk],
+  // phase 2 psi_inv_rev[2^(11-u) + r 2^(3-u) + blk]
+  uint32_t t1[15], t2[15];
+#pragma unroll
+  for (int u = 0; u < 4; u++)
+#pragma unroll
+    for (int blk = 0; blk < (8 >> u); blk++) {
+      t1[16 - (16 >> u) + blk] = w[(32768 >> u) + (r << (7 - u)) + (t << (3 - u)) + blk];
+      t2[16 - (16 >> u) + blk] = w[(2048 >> u) + (r << (3 - u)) + blk];
+    }
+  // twiddles first: with the data in front of them 108 limbs take 16.2 us, not 14.9
+  keep_loads();
+  const uint4 *g = reinterpret_cast<const uint4 *>(J.src + r * 256 + 16 * t);
+  double x[16];
+#pragma unroll
+  for (int i = 0; i < 4; i++) {
+    const uint4 u = g[i];
+    x[4 * i + 0] = (double)u.x;
+    x[4 * i + 1] = (double)u.y;
+    x[4 * i + 2] = (double)u.z;
+    x[4 * i + 3] = (double)u.w;
+  }
+  // sums double every stage: from inputs below 2^31 they stay below 2^39
+  gs16(x, t1, q, qr);
+#pragma unroll
+  for (int j = 0; j < 16; j++) lds[row16_word(rl, 16 * t + j)] = x[j];
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < 16; k++) x[k] = lds[row16_word(rl, t + 16 * k)];
+  gs16(x, t2, q, qr);
+  int32_t *o = reinterpret_cast<int32_t *>(J.dst) + r * 256 + t;
+#pragma unroll
+  for (int k = 0; k < 16; k++) o[16 * k] = lazy_i32(x[k], m);
 }
 
 // ---------------------------------------------------------------------------
@@ -654,6 +751,15 @@ const char *inv_rows_name(int flags) {
 // 59 limbs 24.0 / 23.3 / 23.4; inverse 1 limb 5.1 / 5.4 / 6.4, 24 limbs 13.2 /
 // 12.6 / 13.3, 59 limbs 24.1 / 22.8 / 22.5.
 constexpr int kCols4 = 4, kCols8 = 64;
+// Row pass over n limbs: four values a lane up to these, 16 above. Four / 16
+// values, us, row pass alone: inverse 72 limbs 10.6 / 12.7, 84 limbs 11.9 / 13.5,
+// 96 limbs 14.7 / 14.6, 144 limbs 18.0 / 17.4, 256 limbs 32 / 29, 512 limbs 68 /
+// 57, and 144 limbs within a batch of products 22.8 / 20.0; forward 256 limbs
+// 32.4 / 32.4, 320 limbs 38.7 / 38.5, 384 limbs 48.8 / 45.4, 512 limbs 68 / 61.
+// With a product input (at most 191 limbs) four values stay better: 133 limbs
+// 24.1 / 25.5, 189 limbs 32.4 / 33.2; with the ModDown epilogue the two are equal
+// (506 limbs 75 / 74).
+constexpr int kFwdRows4 = 352, kInvRows4 = 88;
 
 template <class D>
 void fwd_passes(const Context &ctx, const D &d, int n, int flags, hipStream_t st) {
@@ -669,17 +775,29 @@ void fwd_passes(const Context &ctx, const D &d, int n, int flags, hipStream_t st
     else
       cols(ntt_fwd_cols<D>, kColTiles, kColThreads);
   }
-  if (!(flags & kNttColsOnly))
-    launch(ctx, fwd_rows_name(flags), n, ntt_fwd_rows<D>, dim3(kRowTiles, n),
-           dim3(kRowThreads), st, d, ctx.ptab, tw);
+  auto rows = [&](auto kernel, int wgs) {
+    launch(ctx, fwd_rows_name(flags), n, kernel, dim3(wgs, n), dim3(kRowThreads), st, d,
+           ctx.ptab, tw);
+  };
+  if (flags & kNttColsOnly) return;
+  if (n > kFwdRows4 && !(flags & kNttModDownEpilogue))
+    rows(ntt_fwd_rows16<D>, kRow16Tiles);
+  else
+    rows(ntt_fwd_rows<D>, kRowTiles);
 }
 
 template <class D>
 void inv_passes(const Context &ctx, const D &d, int n, int flags,
                 hipStream_t st) {
   const uint32_t *tw = ctx.d_tw_inv;
-  launch(ctx, inv_rows_name(flags), n, intt_rows<D>, dim3(kRowTiles, n), dim3(kRowThreads), st,
-         d, ctx.ptab, tw);
+  auto rows = [&](auto kernel, int wgs) {
+    launch(ctx, inv_rows_name(flags), n, kernel, dim3(wgs, n), dim3(kRowThreads), st, d,
+           ctx.ptab, tw);
+  };
+  if (n > kInvRows4 && !(flags & kInttLoadProduct))
+    rows(intt_rows16<D>, kRow16Tiles);
+  else
+    rows(intt_rows<D>, kRowTiles);
   auto cols = [&](auto kernel, int wgs, int threads) {
     launch(ctx, "intt_cols", n, kernel, dim3(wgs * n), dim3(threads), st, d, ctx.ptab, tw);
   };

@@ -59,3 +59,33 @@ def test_small_transform(params, np3, polys, inverse):
     for k in range(polys):
         assert_same(ck.to_host(dst[k]), want[k], f"call, poly {k}")
         assert_same(ck.to_host(src[k]), want[k], f"call in place, poly {k}")
+
+
+@pytest.mark.parametrize("inverse,mont", [(False, False), (False, True), (True, False),
+                                          (True, True)])
+@pytest.mark.parametrize("params,np3,polys",
+                         [("rns24_aux8.json", (1, 0, 0), 88), ("rns24_aux8.json", (1, 0, 0), 89),
+                          ("rns24_aux8.json", (24, 0, 8), 11), ("bootparam_40.json", (43, 4, 12), 6),
+                          ("rns24_aux8.json", (1, 0, 0), 353)])
+def test_many_limbs(params, np3, polys, inverse, mont):
+    """both sides of the row kernels' lines (88 limbs inverse, 352 forward), in
+    place and not: 16 values a thread above, 16 rows a workgroup"""
+    import cheddar_amd as ck
+    import ckks_oracle as O
+    d = load_params(params)
+    ctx, P = ck.Context.from_json(d), O.Param.from_json(d)
+    O.set_threads(8)
+    ctx.set_plan_forms(ntt="valu")
+    kinds = min(polys, 5)
+    xs = _inputs(P, P.np_primes(*np3), kinds)
+    fn = P.intt_np if inverse else P.ntt_np
+    want = [fn(x, *np3, mont_conv=mont) for x in xs]
+    src = [ck.to_device(xs[k % kinds]) for k in range(polys)]
+    dst = [torch.full_like(s, -1) for s in src]
+    for out in (dst, src):
+        plan = ck.Plan.ntt(ctx, src, out, np3, inverse=inverse, mont_conv=mont)
+        assert plan.info()["form"] == 0
+        plan.run()
+        torch.cuda.synchronize()
+        for k in range(polys):
+            assert_same(ck.to_host(out[k]), want[k % kinds], f"poly {k}")
