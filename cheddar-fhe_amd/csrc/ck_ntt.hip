@@ -745,12 +745,15 @@ const char *inv_rows_name(int flags) {
 
 // Column pass over n limbs. A small launch lasts as long as one wave, so few
 // limbs take four values a thread over four (n <= 4) or eight columns a
-// workgroup, more than 64 the 16-value form. Both passes of a forward transform
+// workgroup, more the 16-value form. Both passes of a forward transform
 // with four columns / eight columns / 16 values, us: 1 limb 5.0 / 5.3 / 6.0,
 // 4 limbs 5.7 / 5.8 / 6.6, 8 limbs 7.1 / 6.9 / 7.6, 24 limbs 12.8 / 12.4 / 12.6,
 // 59 limbs 24.0 / 23.3 / 23.4; inverse 1 limb 5.1 / 5.4 / 6.4, 24 limbs 13.2 /
-// 12.6 / 13.3, 59 limbs 24.1 / 22.8 / 22.5.
-constexpr int kCols4 = 4, kCols8 = 64;
+// 12.6 / 13.3. The inverse line lies lower, since this pass is the lighter one:
+// eight columns / 16 values, the column pass alone, 40 limbs 7.8 / 8.4, 48 limbs
+// 9.2 / 8.8, 56 limbs 10.5 / 10.3, 64 limbs 11.7 / 11.1, and 48 limbs within a batch
+// of products 10.8 / 9.5.
+constexpr int kCols4 = 4, kFwdCols8 = 64, kInvCols8 = 40;
 // Row pass over n limbs: four values a lane up to these, 16 above. Four / 16
 // values, us, row pass alone: inverse 72 limbs 10.6 / 12.7, 84 limbs 11.9 / 13.5,
 // 96 limbs 14.7 / 14.6, 144 limbs 18.0 / 17.4, 256 limbs 32 / 29, 512 limbs 68 /
@@ -770,7 +773,7 @@ void fwd_passes(const Context &ctx, const D &d, int n, int flags, hipStream_t st
     };
     if (n <= kCols4)
       cols(ntt_fwd_cols4<D, 4>, 64, 256);
-    else if (n <= kCols8)
+    else if (n <= kFwdCols8)
       cols(ntt_fwd_cols4<D, 8>, 32, 512);
     else
       cols(ntt_fwd_cols<D>, kColTiles, kColThreads);
@@ -803,7 +806,7 @@ void inv_passes(const Context &ctx, const D &d, int n, int flags,
   };
   if (n <= kCols4)
     cols(intt_cols4<D, 4>, 64, 256);
-  else if (n <= kCols8)
+  else if (n <= kInvCols8)
     cols(intt_cols4<D, 8>, 32, 512);
   else
     cols(intt_cols<D>, kColTiles, kColThreads);

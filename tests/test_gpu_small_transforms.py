@@ -1,8 +1,8 @@
 """GPU parity of the two-pass transforms at the edges of the column kernels'
-rule: four columns a workgroup (to 4 limbs), eight (to 64), 16 values a thread
-above; single calls and plans, both directions, in place and not, primes of 20
-to 31 bits, the residues 0, q - 1, (q - 1) / 2 and (q + 1) / 2 in every limb.
-Whole numbers: every word equals the oracle's."""
+rule: four columns a workgroup (to 4 limbs), eight (to 64, inverse to 40), 16
+values a thread above; single calls and plans, both directions, in place and
+not, primes of 20 to 31 bits, the residues 0, q - 1, (q - 1) / 2 and (q + 1) / 2
+in every limb. Whole numbers: every word equals the oracle's."""
 import pytest
 
 from conftest import SEED_BASE, load_params
@@ -35,6 +35,8 @@ def _inputs(P, pidx, count):
                           ("rns24_aux8.json", (1, 0, 0), 4),
                           ("bootparam_30.json", (5, 0, 0), 1),
                           ("rns24_aux8.json", (24, 0, 8), 2),
+                          ("bootparam_30.json", (40, 0, 0), 1),
+                          ("bootparam_30.json", (41, 0, 0), 1),
                           ("rns24_aux8.json", (5, 0, 8), 5)])
 def test_small_transform(params, np3, polys, inverse):
     import cheddar_amd as ck
