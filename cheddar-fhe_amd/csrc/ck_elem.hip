@@ -441,6 +441,10 @@ __global__ __launch_bounds__(kThreads) void key_accum_table_kernel(
 // XCD windows of eight limbs run chunk by chunk, so that the items of a batch,
 // whose jobs are ordered by prime, read a key's lines from one L2 together.
 //
+// A body per number of groups: one sized for eight re-read group 0 three times
+// for five groups (8 rotations at 29 limbs 133 -> 191 us, six groups at 28 limbs
+// 153 -> 200 us).
+//
 // Bound by memory: 8 rotations of 8 ciphertexts at 8..24 limbs (193 limbs)
 // took 502 us with the scatter and take 320 us, 7 rotations of one at 59 limbs
 // (1.1 GB of keys and outputs) 235 -> 210 us.
@@ -457,9 +461,8 @@ __device__ __forceinline__ BsPlace bs_place() {
                  (w / kBsWindow) * 8 + (int)(blockIdx.x & 7)};
 }
 
-// NG >= ngroups bounds the groups; FULL: equal to it; NT: non-temporal key
-// loads
-template <int NG, bool FULL, bool NT>
+// NG: the number of groups; NT: non-temporal key loads
+template <int NG, bool NT>
 __device__ __forceinline__ void bs_fused_row(const EwNp &np, const PrimeTab &P,
                                              const BsFusedArgs &A, int y, int k,
                                              uint32_t *row) {
@@ -469,21 +472,16 @@ __device__ __forceinline__ void bs_fused_row(const EwNp &np, const PrimeTab &P,
   const size_t my = (size_t)y * 65536 + k;
   const size_t kp = (size_t)p * 65536 + k;
   const size_t tot_stride = (size_t)np.num_total * 65536;
-  const int ng = A.ngroups;
-  // groups past ngroups re-read group 0 and count as zero: all loads are
-  // unconditional and in flight together
   uint32_t mu[NG][4];
 #pragma unroll
   for (int b = 0; b < NG; b++) {
-    const int gi = FULL || b < ng ? b : 0;
-    const bool own = (y >= A.own0[gi] && y < A.own1[gi]);
-    const uint32_t *src = own ? A.x : A.modup + (size_t)A.group[gi] * tot_stride;
+    const bool own = (y >= A.own0[b] && y < A.own1[b]);
+    const uint32_t *src = own ? A.x : A.modup + (size_t)A.group[b] * tot_stride;
     const uint4 v = ld4(src + my);
-    const bool use = FULL || b < ng;
-    mu[b][0] = use ? v.x : 0u;
-    mu[b][1] = use ? v.y : 0u;
-    mu[b][2] = use ? v.z : 0u;
-    mu[b][3] = use ? v.w : 0u;
+    mu[b][0] = v.x;
+    mu[b][1] = v.y;
+    mu[b][2] = v.z;
+    mu[b][3] = v.w;
   }
   uint64_t pb[4] = {0, 0, 0, 0};
   if (y < np.num_q) {
@@ -499,9 +497,8 @@ __device__ __forceinline__ void bs_fused_row(const EwNp &np, const PrimeTab &P,
     uint4 kb[NG], ka[NG];
 #pragma unroll
     for (int b = 0; b < NG; b++) {
-      const int gi = FULL || b < ng ? b : 0;
-      kb[b] = NT ? ld4nt(A.key_b[r][gi] + kp) : ld4(A.key_b[r][gi] + kp);
-      ka[b] = NT ? ld4nt(A.key_a[r][gi] + kp) : ld4(A.key_a[r][gi] + kp);
+      kb[b] = NT ? ld4nt(A.key_b[r][b] + kp) : ld4(A.key_b[r][b] + kp);
+      ka[b] = NT ? ld4nt(A.key_a[r][b] + kp) : ld4(A.key_a[r][b] + kp);
     }
     uint64_t sb[4] = {pb[0], pb[1], pb[2], pb[3]}, sa[4] = {0, 0, 0, 0};
 #pragma unroll
@@ -544,12 +541,16 @@ __device__ __forceinline__ void bs_fused_body(const EwNp &np, const PrimeTab &P,
   const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
   const int k = chunk * kThreads * kVec + (int)threadIdx.x * kVec;
   uint32_t *row = lds + 512 * wave;
+  static_assert(kMaxBsGroups == 8, "a body per number of groups");
   switch (A.ngroups) {
-    case 1: bs_fused_row<1, true, NT>(np, P, A, y, k, row); break;
-    case 2: bs_fused_row<2, true, NT>(np, P, A, y, k, row); break;
-    case 3: bs_fused_row<3, true, NT>(np, P, A, y, k, row); break;
-    case 4: bs_fused_row<4, true, NT>(np, P, A, y, k, row); break;
-    default: bs_fused_row<kMaxBsGroups, false, NT>(np, P, A, y, k, row); break;
+    case 1: bs_fused_row<1, NT>(np, P, A, y, k, row); break;
+    case 2: bs_fused_row<2, NT>(np, P, A, y, k, row); break;
+    case 3: bs_fused_row<3, NT>(np, P, A, y, k, row); break;
+    case 4: bs_fused_row<4, NT>(np, P, A, y, k, row); break;
+    case 5: bs_fused_row<5, NT>(np, P, A, y, k, row); break;
+    case 6: bs_fused_row<6, NT>(np, P, A, y, k, row); break;
+    case 7: bs_fused_row<7, NT>(np, P, A, y, k, row); break;
+    case 8: bs_fused_row<8, NT>(np, P, A, y, k, row); break;
   }
 }
 
