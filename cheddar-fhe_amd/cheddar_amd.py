@@ -448,8 +448,9 @@ class Context:
 
     def set_plan_forms(self, ntt=None, bconv=None, ntt8_blocks=None, ntt8_chunk=None):
         """Forms of ck_plan_ntt forward transforms ("valu", "int8", "auto")
-        and of ck_plan_bconv ("fp64", "int8", "valu", "auto"), and the int8
-        transform's blocks per workgroup / chunk; outputs are identical."""
+        and of ck_plan_bconv ("fp64", "int8", "valu", "auto"), and the two-pass
+        int8 transform's blocks per workgroup / chunk (giving either asks for
+        that form at every size); outputs are identical."""
         if ntt is not None:
             _check(lib.ck_context_set_option(self._h, CK_OPT_PLAN_NTT_FORM, NTT_FORMS[ntt]))
         if bconv is not None:

@@ -1105,8 +1105,11 @@ int ck_plan_ntt(ck_context *ctx, int n, int num_main, int num_ter, int num_aux,
   const int total = n * limbs;
   if (form >= 0) {
     // one pass, unless the two-pass form's shape was chosen by option
-    const bool one_pass = one_pass_limbs(total) > 0 && c.ntt8_blocks == 16 && c.ntt8_chunk == 0;
-    cands.push_back({form, one_pass ? 0 : c.ntt8_blocks, c.ntt8_chunk, -1.0});
+    const bool shaped = c.ntt8_blocks > 0 || c.ntt8_chunk > 0;
+    const int blocks = !shaped && one_pass_limbs(total) > 0 ? 0
+                       : c.ntt8_blocks > 0                  ? c.ntt8_blocks
+                                                            : 16;
+    cands.push_back({form, blocks, c.ntt8_chunk, -1.0});
   } else {
     cands.push_back({0, 0, 0, -1.0});
     if (one_pass_limbs(total) > 0) cands.push_back({1, 0, 0, -1.0});

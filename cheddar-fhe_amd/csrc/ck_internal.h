@@ -178,7 +178,9 @@ struct Context {
   // and CK_OPT_PLAN_BCONV_FORM in cheddar_amd.h (-1: autotune)
   int plan_ntt_form = 1;    // int8 matrix cores (measured faster)
   int plan_bconv_form = 1;  // int8 matrix cores (measured faster)
-  int ntt8_blocks = 16;  // int8 transform: 16-column blocks per workgroup
+  // int8 transform, two-pass form: 16-column blocks per workgroup (0: not set,
+  // 16 where the two-pass form runs; an explicit value asks for that form)
+  int ntt8_blocks = 0;
   int ntt8_chunk = 0;    // int8 transform: limbs per column/row chunk (0: all)
 
   // workspace for multi-kernel operations (one operation at a time per

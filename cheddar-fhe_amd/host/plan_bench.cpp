@@ -7,8 +7,8 @@
 //   plan_bench <params.json> bconv <fp64|int8|valu|auto> [reps]
 //
 // ntt: forward NTT of 64 polynomials x (24 main + 8 auxiliary) limbs, one
-// plan (ck_plan_ntt; blocks / chunk: CK_OPT_NTT8_BLOCKS / CK_OPT_NTT8_CHUNK
-// of the int8 form). bconv: BaseConv of 64 polynomials from the 8 auxiliary
+// plan (ck_plan_ntt; blocks / chunk, when given: CK_OPT_NTT8_BLOCKS /
+// CK_OPT_NTT8_CHUNK of the two-pass int8 form). bconv: BaseConv of 64 polynomials from the 8 auxiliary
 // primes to all 32 (ck_plan_bconv). Inputs are seeded uniform residues
 // (canonical for ntt, centred for bconv) uploaded once; the plan runs once
 // untimed, then `reps` times between two HIP events on one stream. Prints
@@ -66,7 +66,7 @@ int main(int argc, char **argv) {
   }
   const std::string work = argv[2], form = argv[3];
   const int reps = argc > 4 ? std::atoi(argv[4]) : 20;
-  const int blocks = argc > 5 ? std::atoi(argv[5]) : 16;
+  const int blocks = argc > 5 ? std::atoi(argv[5]) : 0;
   const int chunk = argc > 6 ? std::atoi(argv[6]) : 0;
   auto prm = ParameterFromJsonFile(argv[1]);
   const Parameter<uint32_t> &P = *prm;
@@ -114,7 +114,7 @@ int main(int argc, char **argv) {
   ck_plan *plan = nullptr;
   if (is_ntt) {
     if (ck_context_set_option(ctx, CK_OPT_PLAN_NTT_FORM, code) ||
-        ck_context_set_option(ctx, CK_OPT_NTT8_BLOCKS, blocks) ||
+        (blocks && ck_context_set_option(ctx, CK_OPT_NTT8_BLOCKS, blocks)) ||
         ck_context_set_option(ctx, CK_OPT_NTT8_CHUNK, chunk))
       die("options");
     if (ck_plan_ntt(ctx, npoly, nm, 0, na, 0, 0, (const uint32_t *const *)src.data(),

@@ -417,7 +417,7 @@ int ck_plan_destroy(ck_plan *plan);
  * src/core/NTT.cu:231-454); 1 (default, measured faster): the 4-step
  * 256 x 256 transform as exact int8 matrix products (residues split into
  * four bytes, int32 accumulation, exact recombination), in one pass from 192
- * limbs unless CK_OPT_NTT8_BLOCKS or CK_OPT_NTT8_CHUNK is set; -1: autotune,
+ * limbs unless CK_OPT_NTT8_BLOCKS or CK_OPT_NTT8_CHUNK is given; -1: autotune,
  * i.e. build the vector form, the one-pass int8 form (blocks 0) and the
  * two-pass int8 form for every (CK_OPT_NTT8_BLOCKS, CK_OPT_NTT8_CHUNK)
  * candidate, time each and keep the fastest (ck_plan_tuning lists them;
@@ -431,11 +431,13 @@ int ck_plan_destroy(ck_plan *plan);
  * -1: autotune over the three. Results are identical. */
 #define CK_OPT_PLAN_BCONV_FORM 5
 /* CK_OPT_NTT8_BLOCKS: 16-column (16-row) blocks of one limb per workgroup
- * of the int8 transform's column (row) pass: 1, 2, 4, 8 or 16 (default). */
+ * of the two-pass int8 transform's column (row) pass: 1, 2, 4, 8 or 16 (its
+ * default). Setting it, to 16 too, asks for that form at every size. */
 #define CK_OPT_NTT8_BLOCKS 6
 /* CK_OPT_NTT8_CHUNK: limbs per chunk of an int8 transform plan, whose
  * column and row passes run chunk by chunk so that a chunk's intermediate
- * can stay in the last-level cache; 0 (default): one chunk. */
+ * can stay in the last-level cache; 0 (default): one chunk. A chunk size
+ * asks for the two-pass form at every size. */
 #define CK_OPT_NTT8_CHUNK 7
 int ck_context_set_option(ck_context *ctx, int option, int value);
 

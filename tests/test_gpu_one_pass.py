@@ -52,3 +52,25 @@ def test_one_pass(params, np3, polys, launches, inverse, mont):
     torch.cuda.synchronize()
     for k in range(polys):
         assert_same(ck.to_host(dst[k]), want[k % kinds], f"poly {k}")
+
+
+@pytest.mark.parametrize("options,launches", [({}, 1), ({"ntt8_blocks": 16}, 2),
+                                              ({"ntt8_blocks": 4}, 2),
+                                              ({"ntt8_chunk": 512}, 4), ({"ntt8_chunk": 0}, 1)])
+def test_two_pass_form_by_option(rns24, oracle_rns24, options, launches):
+    """1024 limbs (several workgroup rounds): every explicit shape, 16 blocks
+    too, takes the two-pass int8 form"""
+    import cheddar_amd as ck
+    P, np3, polys = oracle_rns24, (24, 0, 8), 32
+    ctx = ck.Context.from_json(rns24)
+    ctx.set_plan_forms(ntt="int8", **options)
+    xs = [uniform(P, P.np_primes(*np3), SEED_BASE + 5700 + k) for k in range(3)]
+    want = [P.ntt_np(x, *np3, mont_conv=True) for x in xs]
+    src = [ck.to_device(xs[k % 3]) for k in range(polys)]
+    dst = [torch.full_like(s, -1) for s in src]
+    plan = ck.Plan.ntt(ctx, src, dst, np3, inverse=False, mont_conv=True)
+    assert plan.info()["launches"] == launches and plan.info()["form"] == 1
+    plan.run()
+    torch.cuda.synchronize()
+    for k in range(polys):
+        assert_same(ck.to_host(dst[k]), want[k % 3], f"poly {k}")
