@@ -1055,6 +1055,14 @@ int ck_plan_ntt(ck_context *ctx, int n, int num_main, int num_ter, int num_aux,
   CK_REQUIRE(form >= 0 || !overlap, "autotuned plans need outputs that do not alias inputs");
   if (overlap) form = 0;
   const int limbs = num_main + num_ter + num_aux;
+  // not set by option: the int8 form where it runs in one pass or its two-pass
+  // shape was given, else the vector passes, which take 10 / 13 / 24 / 38 / 50 us
+  // for 2 / 24 / 64 / 128 / 190 limbs where the two int8 passes take 51 / 51 / 53
+  // / 58 / 59 (a workgroup walks a limb's 16 blocks; with one block a workgroup
+  // 10 / 12 / 23 / 41 / 56)
+  const bool shaped = c.ntt8_blocks > 0 || c.ntt8_chunk > 0;
+  const bool one_pass = !shaped && one_pass_limbs((size_t)n * limbs) > 0;
+  if (form == Context::kNttFormBySize) form = shaped || one_pass ? 1 : 0;
   // large inverse transforms run in one pass on the int8 matrix cores
   const bool inverse_one_pass =
       inverse && !overlap && c.plan_ntt_form != 0 && one_pass_limbs((size_t)n * limbs) > 0;
@@ -1105,10 +1113,7 @@ int ck_plan_ntt(ck_context *ctx, int n, int num_main, int num_ter, int num_aux,
   const int total = n * limbs;
   if (form >= 0) {
     // one pass, unless the two-pass form's shape was chosen by option
-    const bool shaped = c.ntt8_blocks > 0 || c.ntt8_chunk > 0;
-    const int blocks = !shaped && one_pass_limbs(total) > 0 ? 0
-                       : c.ntt8_blocks > 0                  ? c.ntt8_blocks
-                                                            : 16;
+    const int blocks = one_pass ? 0 : c.ntt8_blocks > 0 ? c.ntt8_blocks : 16;
     cands.push_back({form, blocks, c.ntt8_chunk, -1.0});
   } else {
     cands.push_back({0, 0, 0, -1.0});

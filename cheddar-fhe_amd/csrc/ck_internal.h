@@ -176,7 +176,8 @@ struct Context {
   bool fuse_key_rows = true;
   // forms of ck_plan_ntt (forward) and ck_plan_bconv: see CK_OPT_PLAN_NTT_FORM
   // and CK_OPT_PLAN_BCONV_FORM in cheddar_amd.h (-1: autotune)
-  int plan_ntt_form = 1;    // int8 matrix cores (measured faster)
+  static constexpr int kNttFormBySize = 2;  // not set by option
+  int plan_ntt_form = kNttFormBySize;
   int plan_bconv_form = 1;  // int8 matrix cores (measured faster)
   // int8 transform, two-pass form: 16-column blocks per workgroup (0: not set,
   // 16 where the two-pass form runs; an explicit value asks for that form)

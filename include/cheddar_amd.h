@@ -414,11 +414,11 @@ int ck_plan_destroy(ck_plan *plan);
 #define CK_OPT_FUSED_KEY_ROWS 3
 /* CK_OPT_PLAN_NTT_FORM: the form of forward transforms in ck_plan_ntt.
  * 0: radix-16 FP64 butterflies on the vector unit (NTTPhase1 / NTTPhase2,
- * src/core/NTT.cu:231-454); 1 (default, measured faster): the 4-step
- * 256 x 256 transform as exact int8 matrix products (residues split into
- * four bytes, int32 accumulation, exact recombination), in one pass from 192
- * limbs unless CK_OPT_NTT8_BLOCKS or CK_OPT_NTT8_CHUNK is given; -1: autotune,
- * i.e. build the vector form, the one-pass int8 form (blocks 0) and the
+ * src/core/NTT.cu:231-454); 1: the 4-step 256 x 256 transform as exact int8
+ * matrix products (residues split into four bytes, int32 accumulation, exact
+ * recombination), in one pass from 192 limbs unless CK_OPT_NTT8_BLOCKS or
+ * CK_OPT_NTT8_CHUNK is given, else in two; not set (measured fastest): 1
+ * where that is one pass or its shape is given, else 0; -1: autotune, i.e. build the vector form, the one-pass int8 form (blocks 0) and the
  * two-pass int8 form for every (CK_OPT_NTT8_BLOCKS, CK_OPT_NTT8_CHUNK)
  * candidate, time each and keep the fastest (ck_plan_tuning lists them;
  * outputs must not alias inputs). Inverse transforms use the one-pass int8

@@ -74,3 +74,26 @@ def test_two_pass_form_by_option(rns24, oracle_rns24, options, launches):
     torch.cuda.synchronize()
     for k in range(polys):
         assert_same(ck.to_host(dst[k]), want[k % 3], f"poly {k}")
+
+
+@pytest.mark.parametrize("np3,polys,form", [((2, 0, 0), 1, 0), ((24, 0, 0), 1, 0),
+                                            ((13, 0, 8), 9, 0), ((1, 0, 0), 191, 0),
+                                            ((24, 0, 8), 6, 1)])
+def test_forward_form_by_size(rns24, oracle_rns24, np3, polys, form):
+    """nothing set: two vector passes below 192 limbs, one int8 pass from
+    there; the form asked for at every size"""
+    import cheddar_amd as ck
+    P = oracle_rns24
+    xs = [uniform(P, P.np_primes(*np3), SEED_BASE + 5800 + k) for k in range(min(polys, 3))]
+    want = [P.ntt_np(x, *np3, mont_conv=True) for x in xs]
+    src = [ck.to_device(xs[k % 3]) for k in range(polys)]
+    for asked, got in ((None, form), ("int8", 1), ("valu", 0)):
+        ctx = ck.Context.from_json(rns24)
+        ctx.set_plan_forms(ntt=asked)
+        dst = [torch.full_like(s, -1) for s in src]
+        plan = ck.Plan.ntt(ctx, src, dst, np3, inverse=False, mont_conv=True)
+        assert plan.info()["form"] == got and plan.info()["launches"] == (1 if got and form else 2)
+        plan.run()
+        torch.cuda.synchronize()
+        for k in range(polys):
+            assert_same(ck.to_host(dst[k]), want[k % 3], f"{asked}, poly {k}")
