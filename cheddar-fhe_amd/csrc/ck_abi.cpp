@@ -744,25 +744,39 @@ int ck_hrot_hoisted(ck_context *ctx, int level, int n_rot, const int *rots,
 // both key passes (the ModUp's row stages fused with the key inner product,
 // or a row pass plus a separate accumulation): times each and keeps the
 // fastest. build(bconv form, key pass (-1: the context's), item chunks
-// (0: the builder's default), &plan). With chunk_items > 0 (HMult plans),
-// the fastest form is then also built with its items in 2, 4 and 8 chunks
-// (at least two items each) and the fastest of those kept.
+// (0: the builder's default), &plan). The plan that would be built without
+// tuning is a candidate too: the order of the forms with all items in one
+// chunk is not their order in several (64 HMults at 8..24 limbs: FP64 form 2.63
+// ms and fused 2.66 in one chunk, fused 2.25 in four). With chunk_items > 0 (HMult
+// plans), the fastest form is then also built with its items in 2, 4 and 8
+// chunks (at least two items each) and the fastest of those kept.
 extern "C++" template <typename Build>
 static int build_tuned(const Context &c, Build &build, bool key_dim, int chunk_items,
                        Plan **out) {
   *out = nullptr;
-  if (!c.plan_autotune) return build(c.bconv_mfma < 0 ? 0 : c.bconv_mfma, -1, 0, out);
+  const int untuned = c.bconv_mfma < 0 ? 0 : c.bconv_mfma;
+  if (!c.plan_autotune) return build(untuned, -1, 0, out);
   Plan *best = nullptr;
   double best_us = -1.0;
   double us[3] = {-1.0, -1.0, -1.0};
   std::vector<Plan::Candidate> rec;
   int best_f = 0, best_kr = -1;
+  auto key_pass = [&](int kr) { return kr < 0 ? (c.fuse_key_rows ? 1 : 0) : kr; };
+  auto known = [&](int f, int kr, int chunks) {
+    for (const Plan::Candidate &r : rec)
+      if (r.form == f && r.blocks == key_pass(kr) && r.chunk == chunks) return true;
+    return false;
+  };
   auto consider = [&](int f, int kr, int chunks) -> int {
     Plan *p = nullptr;
     int rc = build(f, kr, chunks, &p);
     if (rc) return rc;
+    if (chunks != 1 && known(f, kr, p->chunks)) {
+      plan_destroy(p);
+      return kOk;
+    }
     const double t = plan_time_us(*p, 3);
-    rec.push_back({f, kr < 0 ? (c.fuse_key_rows ? 1 : 0) : kr, p->chunks, t});
+    rec.push_back({f, key_pass(kr), p->chunks, t});
     if (t >= 0 && (us[f] < 0 || t < us[f])) us[f] = t;
     if (t >= 0 && (!best || t < best_us)) {
       plan_destroy(best);
@@ -783,10 +797,15 @@ static int build_tuned(const Context &c, Build &build, bool key_dim, int chunk_i
         return rc;
       }
     }
+  int rc = consider(untuned, -1, 0);
+  if (rc) {
+    plan_destroy(best);
+    return rc;
+  }
   if (best)
     for (int k : {2, 4, 8}) {
       if (chunk_items < 2 * k) break;
-      const int rc = consider(best_f, best_kr, k);
+      rc = consider(best_f, best_kr, k);
       if (rc) {
         plan_destroy(best);
         return rc;

@@ -400,8 +400,9 @@ int ck_plan_destroy(ck_plan *plan);
 /* CK_OPT_PLAN_AUTOTUNE: 1 makes ck_plan_hmult / ck_plan_hrot_hoisted build
  * the plan with each BaseConv form (fused, FP64 matrix cores, int8 matrix
  * cores; for ck_plan_hmult each with both key passes, CK_OPT_FUSED_KEY_ROWS
- * 1 and 0, all in one chunk, then the fastest of those in 2, 4 and 8 item
- * chunks), run each (one warm-up + 3 timed runs on a private stream,
+ * 1 and 0, all in one chunk, then the plan that 0 builds, where that has
+ * several item chunks, then the fastest of those in 2, 4 and 8 chunks), run
+ * each (one warm-up + 3 timed runs on a private stream,
  * synchronising the host: plan creation only; the runs write the plan's
  * outputs) and keep the fastest (ck_plan_tuning lists the times); 0
  * (default) uses CK_OPT_BCONV_MFMA and the default chunks. */
@@ -418,12 +419,13 @@ int ck_plan_destroy(ck_plan *plan);
  * matrix products (residues split into four bytes, int32 accumulation, exact
  * recombination), in one pass from 192 limbs unless CK_OPT_NTT8_BLOCKS or
  * CK_OPT_NTT8_CHUNK is given, else in two; not set (measured fastest): 1
- * where that is one pass or its shape is given, else 0; -1: autotune, i.e. build the vector form, the one-pass int8 form (blocks 0) and the
- * two-pass int8 form for every (CK_OPT_NTT8_BLOCKS, CK_OPT_NTT8_CHUNK)
- * candidate, time each and keep the fastest (ck_plan_tuning lists them;
- * outputs must not alias inputs). Inverse transforms use the one-pass int8
- * form from 192 limbs (unless 0 is set), else the vector form. Results are
- * identical. */
+ * where that is one pass or its shape is given, else 0; -1: autotune, i.e.
+ * build the vector form, the one-pass int8 form (blocks 0) and the two-pass
+ * int8 form for every (CK_OPT_NTT8_BLOCKS, CK_OPT_NTT8_CHUNK) candidate, time
+ * each and keep the fastest (ck_plan_tuning lists them; outputs must not
+ * alias inputs). Inverse transforms are not tuned: they use the one-pass
+ * int8 form from 192 limbs (unless 0 is set), else the vector form. Results
+ * are identical. */
 #define CK_OPT_PLAN_NTT_FORM 4
 /* CK_OPT_PLAN_BCONV_FORM: the form of ck_plan_bconv. 0: FP64 matrix cores
  * (16-bit table halves); 1 (default, measured faster): int8 matrix cores

@@ -155,6 +155,38 @@ def test_plan_graph_replays(ck, ctx24, oracle_rns24, key24):
                 assert torch.equal(outs[i][k], eager[i][k]), (rep, i, k)
 
 
+def test_autotuning_times_the_untuned_plan(ck, rns24):
+    """a batch whose default plan has three item chunks, a number that the
+    search over chunks (1, 2, 4, 8) does not try: that plan is among the
+    candidates, each candidate once, the fastest is kept, same outputs"""
+    ctx = ck.Context.from_json(rns24)
+    gen = torch.Generator(device="cuda").manual_seed(SEED_BASE % 2**31)
+    n, level = 24, 23
+    q = ctx.num_q(level)
+
+    def poly(limbs):
+        return torch.randint(0, 2**19, (limbs, ctx.n), dtype=torch.int32, device="cuda",
+                             generator=gen)
+    ct1, ct2 = ([[poly(q) for _ in range(2)] for _ in range(n)] for _ in range(2))
+    key = tuple([poly(ctx.num_primes) for _ in range(ctx.dnum)] for _ in range(2))
+    outs = [[[torch.empty((q - 1, ctx.n), dtype=torch.int32, device="cuda") for _ in range(2)]
+             for _ in range(n)] for _ in range(2)]
+    plan = ck.Plan.hmult(ctx, [level] * n, outs[0], ct1, ct2, key)
+    plan.run()
+    ctx.set_plan_autotune(True)
+    tuned = ck.Plan.hmult(ctx, [level] * n, outs[1], ct1, ct2, key)
+    tuning = tuned.tuning()
+    shapes = [t[:3] for t in tuning]
+    assert (0, 1, 3) in shapes and len(set(shapes)) == len(shapes)
+    best = min(tuning, key=lambda t: t[3])
+    assert (tuned.info()["bconv_form"], tuned.info()["form"]) == \
+        (("fused", "fp64", "int8")[best[0]], best[1])
+    tuned.run()
+    torch.cuda.synchronize()
+    for x, y in zip(outs[0], outs[1]):
+        assert torch.equal(x[0], y[0]) and torch.equal(x[1], y[1])
+
+
 def test_autotuned_plans_reject_aliasing(ck, rns24, oracle_rns24, key24):
     """the timed candidate runs of an autotuned plan write its outputs, so
     outputs that alias inputs are refused at plan creation"""
