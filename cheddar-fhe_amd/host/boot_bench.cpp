@@ -14,8 +14,8 @@
 //
 // sse (default): the file's dense Hamming weight with sparse-secret
 // encapsulation; nosse: the main secret gets the sparse weight. bconv: the
-// CK_OPT_BCONV_MFMA value (-1 default, 0 fused, 1 FP64, 2 int8 matrix
-// cores). lanes (default 4): contexts of the graph, bootstrap i on lane
+// CK_OPT_BCONV_MFMA value (-1 default, 0 fused with the forward column pass, 1
+// FP64 and 2 int8 matrix cores as a step of its own). lanes (default 4): contexts of the graph, bootstrap i on lane
 // i mod lanes, each lane a stream of its own.
 #include <algorithm>
 #include <chrono>
