@@ -987,6 +987,7 @@ uint32_t brv_n(uint32_t x, int bits) {
 }  // namespace
 
 int ntt8_tables(Context &c, I8NttTabs *out) {
+  std::lock_guard<std::mutex> lock(c.tables_mu);
   if (c.i8_planes) {
     *out = I8NttTabs{c.i8_planes, c.i8_corr, c.i8_tw, c.i8_twm};
     return kOk;
@@ -1081,6 +1082,7 @@ int ntt8_tables(Context &c, I8NttTabs *out) {
 // twm: psi^(-c (2 brv8(p) + 1)) 2^32, centred, for column c = c0 + 16 (4 g + v)
 // and row p = s + 16 n at word ((16 c0 + s) 64 + 16 g + n) 4 + v.
 int ntt1p_inv_tables(Context &c, I8InvTabs *out) {
+  std::lock_guard<std::mutex> lock(c.tables_mu);
   if (c.i8_inv_planes) {
     *out = I8InvTabs{c.i8_inv_planes, c.i8_inv_corr, c.i8_inv_twm};
     return kOk;
@@ -1207,6 +1209,7 @@ void launch_bconv_i8(const Context &c, const BconvI8Launch &L, hipStream_t st) {
 
 const int64_t *bconv_i8_planes_for(const Context &c, const double *d_ftab, int S, int D,
                                    const uint8_t *dst_prime) {
+  std::lock_guard<std::mutex> lock(c.tables_mu);
   for (auto &e : c.i8_bconv_planes)
     if (e.first == d_ftab) return e.second;
   std::vector<double> f((size_t)2 * S * D);

@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -190,6 +191,9 @@ struct Context {
   size_t ws_words = 0;
 
   std::vector<void *> allocations;
+  // held while the tables that plans build on first use are looked up or built
+  // (i8_*): plans of one context may be created by several host threads
+  mutable std::mutex tables_mu;
 
   // optional per-kernel timing: HIP events recorded around every launch on
   // the caller's stream while enabled (ck_profile_*)

@@ -97,3 +97,39 @@ def test_forward_form_by_size(rns24, oracle_rns24, np3, polys, form):
         torch.cuda.synchronize()
         for k in range(polys):
             assert_same(ck.to_host(dst[k]), want[k % 3], f"{asked}, poly {k}")
+
+
+def test_plans_created_by_several_threads(rns24, oracle_rns24):
+    """a fresh context's first plans, forward and inverse, from four threads at
+    once: the tables they share are built once"""
+    import threading
+
+    import cheddar_amd as ck
+    P, np3, polys = oracle_rns24, (24, 0, 8), 6
+    ctx = ck.Context.from_json(rns24)
+    x = uniform(P, P.np_primes(*np3), SEED_BASE + 5900)
+    src = [ck.to_device(x) for _ in range(polys)]
+    dst = [[torch.full_like(s, -1) for s in src] for _ in range(4)]
+    plans, errors, start = [None] * 4, [], threading.Barrier(4)
+
+    def build(i):
+        try:
+            start.wait()
+            plans[i] = ck.Plan.ntt(ctx, src, dst[i], np3, inverse=bool(i & 1), mont_conv=True)
+        except Exception as e:  # reported by the main thread
+            errors.append(e)
+
+    threads = [threading.Thread(target=build, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors
+    for p in plans:
+        assert p.info()["launches"] == 1
+        p.run()
+    torch.cuda.synchronize()
+    for i in range(4):
+        want = (P.intt_np if i & 1 else P.ntt_np)(x, *np3, mont_conv=True)
+        for k in range(polys):
+            assert_same(ck.to_host(dst[i][k]), want, f"thread {i} poly {k}")
