@@ -90,9 +90,10 @@ __device__ __forceinline__ int32_t centre(uint32_t a, uint32_t q) {
 // 2.4 GHz, an FP64 multiply-add 5.4), so a sum costs a fraction of reducing
 // every product.
 
-// a < q 2^32 -> a minus a multiple of q 2^32, in [0, q 2^32), for the sum of
-// such a value and two products of residues (a < 2 q 2^32 < 2^64: each product
-// is below q^2 < q 2^31)
+// a < 2 q 2^32 -> a or a - q 2^32, in [0, q 2^32). At most two products of
+// residues may be added to a folded value before the next fold: each is below
+// q^2 < q 2^31, so that the sum stays below 2 q 2^32 < 2^64, and a third would
+// not; up to four may be summed from zero.
 __device__ __forceinline__ uint64_t sum_fold(uint64_t a, uint32_t q) {
   const uint32_t hi = (uint32_t)(a >> 32), h2 = hi - q;
   return ((uint64_t)(hi < h2 ? hi : h2) << 32) | (uint32_t)a;

@@ -54,12 +54,6 @@ __device__ __forceinline__ void st1(uint32_t *p, uint32_t v) {
   *(__attribute__((address_space(1))) uint32_t *)p = v;
 }
 
-// compile-time count tag for the per-count bodies below
-template <int N>
-struct IntC {
-  static constexpr int value = N;
-};
-
 template <typename F>
 __device__ __forceinline__ uint4 map2(uint4 a, uint4 b, F f) {
   return make_uint4(f(a.x, b.x), f(a.y, b.y), f(a.z, b.z), f(a.w, b.w));
