@@ -1,6 +1,7 @@
 """GPU parity of the one-pass int8 transforms at the edges of their rule:
 the smallest batch that takes them, whole rounds of 256 limbs, a short last
-round (two vector passes) and a long one, both directions, both Montgomery
+round (two vector passes: 1, 5, 64, 65 and 127 limbs, both sides of the column
+kernels' lines) and a long one (128), both directions, both Montgomery
 options, primes of 20 to 31 bits, the residues 0, q - 1, (q - 1) / 2 and
 (q + 1) / 2 in every limb. Whole numbers: every word equals the oracle's."""
 import numpy as np
@@ -18,6 +19,10 @@ torch = pytest.importorskip("torch")
                          [("rns24_aux8.json", (24, 0, 8), 6, 1),
                           ("rns24_aux8.json", (16, 0, 0), 16, 1),
                           ("rns24_aux8.json", (1, 0, 0), 257, 3),
+                          ("rns24_aux8.json", (9, 0, 0), 29, 3),
+                          ("rns24_aux8.json", (24, 0, 8), 10, 3),
+                          ("rns24_aux8.json", (3, 0, 0), 107, 3),
+                          ("rns24_aux8.json", (1, 0, 0), 383, 3),
                           ("rns24_aux8.json", (24, 0, 8), 12, 1),
                           ("rns24_aux8.json", (17, 0, 0), 11, 2),
                           ("bootparam_40.json", (43, 4, 12), 4, 1),
@@ -46,7 +51,7 @@ def test_one_pass(params, np3, polys, launches, inverse, mont):
     dst = [torch.full_like(s, -1) for s in src]
     plan = ck.Plan.ntt(ctx, src, dst, np3, inverse=inverse, mont_conv=mont)
     limbs = polys * sum(np3)
-    # 187 limbs: below the rule, the two passes of either form
+    # 187 limbs: below the rule, two vector passes
     assert plan.info()["launches"] == launches, limbs
     plan.run()
     torch.cuda.synchronize()

@@ -1,7 +1,7 @@
 """GPU parity of the two-pass transforms at the edges of the column kernels'
 rule: four columns a workgroup (to 4 limbs), eight (to 64, inverse to 40), 16
-values a thread above; single calls and plans, both directions, in place and
-not, primes of 20 to 31 bits, the residues 0, q - 1, (q - 1) / 2 and (q + 1) / 2
+values a thread above; single calls and plans, both directions, both Montgomery
+options, in place and not, primes of 20 to 31 bits, the residues 0, q - 1, (q - 1) / 2 and (q + 1) / 2
 in every limb. Whole numbers: every word equals the oracle's."""
 import pytest
 
@@ -25,7 +25,8 @@ def _inputs(P, pidx, count):
     return xs
 
 
-@pytest.mark.parametrize("inverse", [False, True])
+@pytest.mark.parametrize("inverse,mont", [(False, False), (False, True), (True, False),
+                                          (True, True)])
 @pytest.mark.parametrize("params,np3,polys",
                          [("rns24_aux8.json", (1, 0, 0), 1),
                           ("bootparam_40.json", (1, 1, 2), 1),
@@ -38,7 +39,7 @@ def _inputs(P, pidx, count):
                           ("bootparam_30.json", (40, 0, 0), 1),
                           ("bootparam_30.json", (41, 0, 0), 1),
                           ("rns24_aux8.json", (5, 0, 8), 5)])
-def test_small_transform(params, np3, polys, inverse):
+def test_small_transform(params, np3, polys, inverse, mont):
     import cheddar_amd as ck
     import ckks_oracle as O
     d = load_params(params)
@@ -46,17 +47,20 @@ def test_small_transform(params, np3, polys, inverse):
     O.set_threads(8)
     xs = _inputs(P, P.np_primes(*np3), polys)
     fn = P.intt_np if inverse else P.ntt_np
-    want = [fn(x, *np3, mont_conv=inverse) for x in xs]
+    want = [fn(x, *np3, mont_conv=mont) for x in xs]
     src = [ck.to_device(x) for x in xs]
     dst = [torch.full_like(s, -1) for s in src]
-    ck.Plan.ntt(ctx, src, dst, np3, inverse=inverse, mont_conv=inverse).run()
+    ctx.set_plan_forms(ntt="valu")
+    plan = ck.Plan.ntt(ctx, src, dst, np3, inverse=inverse, mont_conv=mont)
+    assert plan.info()["form"] == 0 and plan.info()["launches"] == 2
+    plan.run()
     torch.cuda.synchronize()
     for k in range(polys):
         assert_same(ck.to_host(dst[k]), want[k], f"plan, poly {k}")
     call = ctx.intt if inverse else ctx.ntt
     for k in range(polys):
-        call(dst[k], src[k], *np3, mont_conv=inverse)
-        call(src[k], src[k], *np3, mont_conv=inverse)
+        call(dst[k], src[k], *np3, mont_conv=mont)
+        call(src[k], src[k], *np3, mont_conv=mont)
     torch.cuda.synchronize()
     for k in range(polys):
         assert_same(ck.to_host(dst[k]), want[k], f"call, poly {k}")

@@ -17,13 +17,13 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-ffp-contract=off",
          "--cuda-device-only", "-c", "-o", os.devnull,
          "-Rpass-analysis=kernel-resource-usage"]
 
-# minimum waves per SIMD for the transform passes (LDS allows five); the
-# column pass's instantiations for BaseConv over 10..16 sources (mangled
-# with template argument Li1E) and 17..24 sources (Li2E) are built for four
-# and three
+# minimum waves per SIMD: the transform passes (LDS allows five), the column
+# pass with BaseConv (two workgroups of eight waves on a CU), the key products
+# and the hoisted baby steps (their keys' loads in flight), the one-pass
+# transforms (one workgroup of eight waves on a CU)
 MIN_OCCUPANCY = {"ntt_fwd_cols": 5, "ntt_fwd_rows": 5, "intt_rows": 5, "intt_cols": 5,
-                 "ntt8_cols": 3, "ntt8_rows": 3}
-WIDE_OCCUPANCY = {"Li1E": 4, "Li2E": 3}
+                 "ntt8_cols": 3, "ntt8_rows": 3, "bconv_i8_cols": 4, "key_rows": 5,
+                 "bs_fused": 4, "ntt1p_fwd": 2, "ntt1p_inv": 2}
 
 
 def extra_flags(src):
@@ -62,8 +62,4 @@ def test_no_spills_and_occupancy(src):
         assert r.get("ScratchSize", 0) == 0, (fn, r)
         for k, occ in MIN_OCCUPANCY.items():
             if k in fn:
-                if k == "ntt_fwd_cols":
-                    for tag, o in WIDE_OCCUPANCY.items():
-                        if tag in fn:
-                            occ = o
                 assert r.get("Occupancy", 0) >= occ, (fn, r)
