@@ -75,11 +75,13 @@ def alg_limbs(ctx, level, name):
 
 
 def kernel_key(name):
-    """'ntt_fwd_cols+bconv/72' -> 'ntt_fwd_cols/72': the kernel symbol and
+    """'ntt_fwd_rows+epilogue/46' -> 'ntt_fwd_rows/46': the kernel symbol and
     its limb count, the key rocprof summaries use."""
     kern, n = name.rsplit("/", 1)
     if kern == "ntt_fwd_rows+key":
         return f"key_rows/{n}"
+    if kern == "ntt_fwd_cols+bconv":  # whole quads of destinations
+        return f"bconv_i8_cols/{-(-int(n) // 4) * 4}"
     return f"{kern.split('+')[0]}/{n}"
 
 
@@ -100,7 +102,8 @@ def measured_traffic(kernel):
 # Launch grids -> limb counts: column passes run 16 workgroups per limb with 16
 # values a thread, 32 or 64 with four (by their size, 512 or 256 threads); row
 # passes 64 per limb or, with 16 values a thread, 16 (grid y = limbs),
-# element-wise kernels 64.
+# element-wise kernels 64. The column pass with BaseConv is labelled by four limbs
+# a quad of destinations: 256 columns over the 8 or 16 of a workgroup, a wave each.
 def _short(sym):
     s = sym.replace("void ", "").replace("ck::(anonymous namespace)::", "")
     s = s.replace("ck::", "").split("(")[0]
@@ -115,8 +118,11 @@ _KERNELS = ("ntt_fwd_cols", "intt_cols", "ntt_fwd_cols4", "intt_cols4", "ntt_fwd
             "key_rows_table", "gs_accum")
 # int8 matrix-core kernels (batched plans): labelled by workgroup count, since
 # their workgroups per limb depend on the plan's blocks per workgroup
-_I8_KERNELS = ("ntt8_cols", "ntt8_rows", "ntt1p_fwd", "ntt1p_inv", "bconv_i8", "bconv_valu",
-               "bconv_i8_cols")
+_I8_KERNELS = ("ntt8_cols", "ntt8_rows", "ntt1p_fwd", "ntt1p_inv", "bconv_i8", "bconv_valu")
+
+
+def _quad_limbs(wgs, wg_x):
+    return wgs * (wg_x // 64) // 256 * 4
 
 
 def _limbs(short, grid_x, grid_y, wg_x):
@@ -125,6 +131,8 @@ def _limbs(short, grid_x, grid_y, wg_x):
     wgs = grid_x // max(1, wg_x)
     if short in _I8_KERNELS:
         return f"{wgs}wg"
+    if short == "bconv_i8_cols":
+        return _quad_limbs(wgs, wg_x)
     if short == "copy16":  # ck_copy: 16 bytes per thread, labelled by size
         return f"{(wgs * wg_x * 16) >> 20}MiB"
     if short not in _KERNELS:
@@ -191,6 +199,10 @@ def pmc_traffic(fetch_csv, write_csv, scale=None):
                 n = grid // wg // 64
             elif short in ("ntt_fwd_rows16", "intt_rows16"):
                 n = grid // wg // 16
+            elif short == "bconv_i8_cols":
+                n = _quad_limbs(grid // wg, wg)
+            elif short in ("ntt1p_fwd", "ntt1p_inv"):
+                n = grid // wg  # a workgroup a limb
             elif short in ("key_accum", "tensor", "permute"):
                 n = grid // wg // 64
             elif short in ("gs_accum", "permute_accum"):
@@ -458,9 +470,9 @@ def main():
                     help="print a per-kernel summary of a rocprofv3 --kernel-trace "
                          "CSV and exit")
     ap.add_argument("--bconv", choices=("auto", "fused", "mfma"), default="auto",
-                    help="BaseConv fused into the forward NTT column pass, on the FP64 "
-                         "matrix cores as its own step, or auto (matrix cores in batched "
-                         "plans only)")
+                    help="BaseConv fused with the forward NTT column pass on the int8 "
+                         "matrix cores (also auto, unless plans are tuned), or on the FP64 "
+                         "matrix cores as its own step")
     ap.add_argument("--workload", choices=("hmult", "batched"), default="hmult",
                     help="hmult: one HMult+relin+rescale per step at L=24 (default); "
                          "batched: 64 ciphertexts at 8..24 limbs through one HMult "

@@ -64,3 +64,27 @@ def test_pmc_traffic_calibration_copy(tmp_path):
     _write(f, "FETCH_SIZE", [(GS, 8 * 32768, 64.0)])
     with pytest.raises(SystemExit):
         b.pmc_traffic(str(f), str(w))
+
+
+def test_labels_of_the_transform_kernels(tmp_path):
+    """one label per kernel and limb count, whatever a workgroup holds"""
+    b = _bench()
+    ns = "void ck::(anonymous namespace)::"
+    rows = [(ns + "bconv_i8_cols<ck::BcolsByValue, 8, 0>(x)", 18 * 32, 512, "bconv_i8_cols/72"),
+            (ns + "bconv_i8_cols<ck::BcolsTable, 16, 1>(x)", 12 * 16, 1024, "bconv_i8_cols/48"),
+            (ns + "ntt_fwd_rows16<ck::JobTable>(x)", 16 * 400, 256, "ntt_fwd_rows16/400"),
+            (ns + "intt_rows<ck::JobByValue>(x)", 64 * 24, 256, "intt_rows/24"),
+            (ns + "intt_cols4<ck::JobByValue, 8>(x)", 32 * 24, 512, "intt_cols4/24"),
+            (ns + "ntt1p_fwd_kernel(x)", 256, 512, "ntt1p_fwd/256"),
+            (ns + "key_rows_kernel(x)", 64 * 32, 256, "key_rows/32")]
+    for path, counter in (("f.csv", "FETCH_SIZE"), ("w.csv", "WRITE_SIZE")):
+        with open(tmp_path / path, "w", newline="") as f:
+            w = csv.DictWriter(f, fieldnames=FIELDS)
+            w.writeheader()
+            for name, wgs, wg, _ in rows:
+                w.writerow({"Kernel_Name": name, "Grid_Size": wgs * wg, "Workgroup_Size": wg,
+                            "Counter_Name": counter, "Counter_Value": 1.0})
+    out = b.pmc_traffic(str(tmp_path / "f.csv"), str(tmp_path / "w.csv"), scale=(2.0, 1.0))
+    assert set(out["kernels"]) == {r[3] for r in rows}
+    assert b.kernel_key("ntt_fwd_cols+bconv/46") == "bconv_i8_cols/48"
+    assert b.kernel_key("ntt_fwd_rows+key/32") == "key_rows/32"
