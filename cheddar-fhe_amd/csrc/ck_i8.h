@@ -52,8 +52,10 @@ void launch_ntt8_rows(const Context &c, const I8NttTabs &T, const Ntt8Job *jobs,
 // takes it; of the limbs past its whole rounds, 128 and more too, fewer run
 // as two passes (7.5 us and 0.25 us a limb). Measured for 192 / 256 / 512 /
 // 2048 limbs, against two vector passes: forward 38 / 37 / 74 / 318 us against
-// 55 / 64 / 129 / 570, inverse 42 / 40 / 78 / 334 us against 52 / 62 / 120 /
-// 543; at 264 limbs a second round for 8 of them costs 63 and 70 us in all.
+// 49 / 62 / 126 / 559, inverse 42 / 40 / 78 / 334 us against 47 / 60 / 120 /
+// 544; at 264 limbs a second round for 8 of them costs 63 and 70 us in all.
+// With the product input a round takes 53 us at 192 limbs and 57-60 at 240 to
+// 256, against 60 and 73-75 of the two vector passes.
 constexpr int kOnePassLimbs = 192, kOnePassRound = 256, kOnePassTail = 128;
 inline size_t one_pass_limbs(size_t n) {  // how many of n limbs, the first ones
   if (n < (size_t)kOnePassLimbs) return 0;

@@ -1292,6 +1292,11 @@ void bconv_cols_nc(const Context &c, const D &d, int n, int limbs, int max_s, hi
 // sources the loads weigh more and whole 64-byte segments win once ten quads
 // fill the chip: 42 limbs of 15 sources 14.5 against 16.9 us, 114 of 12
 // sources 23.5 against 24.5 us; 4 limbs of 9 sources 10.2 against 7.5 us.
+// Nine sources lie on the line: with 16 / 8 columns 28 limbs of 8 polynomials
+// 10.8 / 12.1 us, 48 limbs of 6 12.0 / 13.3, 192 limbs of 128 65.6 / 82.4, but 92
+// limbs of 4 23.5 / 19.8, 254 limbs of 12 51.5 / 44.7, 506 limbs of 22 90 / 81: a
+// polynomial's quads share its sources in a cache, which the few limbs of the
+// first three do not.
 template <class D>
 void bconv_cols(const Context &c, const D &d, int n, int limbs, int max_s, hipStream_t st) {
   if (n <= 0) return;

@@ -11,9 +11,10 @@
 // MI355X mapping. A limb of 2^16 u32 is a 256 x 256 matrix (row = 256
 // consecutive coefficients).
 //   * row kernels (forward stages 8..15, inverse stages 0..7): a wave owns one
-//     row, four values a lane, without a barrier; the transformed side moves
-//     with 16-byte accesses, the other with 4-byte accesses over 256
-//     contiguous bytes.
+//     row, four values a lane, without a barrier, or for many limbs a
+//     workgroup 16 rows, 16 values a thread; the transformed side moves with
+//     16-byte accesses, the other with 4-byte accesses over 256 (or four times
+//     64) contiguous bytes.
 //   * column kernels (forward stages 0..7, inverse 8..15): a workgroup owns all
 //     256 rows of 4, 8 or 16 columns (four values a thread, or 16 at 16
 //     columns), read and written straight from registers.
