@@ -1060,9 +1060,9 @@ int ck_plan_ntt(ck_context *ctx, int n, int num_main, int num_ter, int num_aux,
   CK_REQUIRE(n >= 1, "a plan needs at least one polynomial");
   CK_REQUIRE(valid_np(c, num_main, num_ter, num_aux), "invalid NP");
   for (int k = 0; k < n; k++) CK_REQUIRE(src[k] && dst[k], "null pointer");
-  // the int8 matrix-core form covers the forward transform; its column pass
-  // writes a tiled intermediate over dst, which must therefore not overlap
-  // any input: in-place plans take the vector form
+  // the column pass of the two-pass int8 form writes a tiled intermediate over
+  // dst, which must therefore not overlap any input: in-place plans take the
+  // vector form
   bool overlap = false;
   const size_t bytes = (size_t)(num_main + num_ter + num_aux) * kLimb * sizeof(uint32_t);
   for (int k = 0; k < n && !overlap; k++)

@@ -360,9 +360,11 @@ int ck_plan_bconv(ck_context *ctx, const int *src_primes, int n_src,
                   uint32_t *const *dst, ck_plan **out);
 /* dst[k] = ck_ntt (inverse = 0) or ck_intt (inverse = 1) of src[k], k < n,
  * all with one NP (NTTHandler::NTT / INTT over a batch): one launch per pass
- * across the batch. From 192 limbs the int8 form runs in one pass, both ways.
- * Its two-pass form writes a tiled intermediate over dst, so a plan whose
- * outputs overlap its inputs (in place) uses the vector form. */
+ * across the batch. From 192 limbs the int8 form runs in one pass, both ways;
+ * smaller batches take two vector passes unless a form is asked for
+ * (CK_OPT_PLAN_NTT_FORM). The two-pass int8 form writes a tiled intermediate
+ * over dst, so a plan whose outputs overlap its inputs (in place) uses the
+ * vector form. */
 int ck_plan_ntt(ck_context *ctx, int n, int num_main, int num_ter, int num_aux,
                 int inverse, int montgomery_conversion, const uint32_t *const *src,
                 uint32_t *const *dst, ck_plan **out);
